@@ -165,6 +165,35 @@ int rwkv6_shift_lerp_bwd(const void* x, const void* maa, int param_dtype, const 
                          void* workspace, int64_t T, int64_t B, int64_t C, void* stream);
 
 /* ------------------------------------------------------------------------
+ * The two bottlenecks of RWKV6TimeMix end to end (RWKV6Bottleneck.forward,
+ * rwkv6_layer_specs.py:177-195, at :440-452 and :454), weights as the module holds them:
+ * w_down [C, E*R], w_up [E*R, C] in w_dtype, bias [E, C] in bias_dtype.  Two forms:
+ *   maa (and x of the up call) given:  E = 5, R = 32, on xxx = x + (shift(x) - x) * maa, the five
+ *       mixes x + (shift(x) - x) * (neck_e @ w_up[e] + bias[e]) as outputs;
+ *   maa (x of the up call) NULL:       E = 1, R = 64, out = neck @ w_up + bias.
+ * Other E, R return RWKV6_ERR_UNSUPPORTED (rwkv6_shift_lerp_fwd / rwkv6_ddlerp_lora_* /
+ * rwkv6_lora_bias_fwd and GEMMs cover them).  C must be a multiple of 64.
+ *   down: neck [N, E*R] bf16 = tanh(xxx @ w_down)   (or x @ w_down)
+ *   up:   out = host array of E device pointers, [T,B,C] bf16 each
+ *   bwd:  d_out = host array of E device pointers [T,B,C] bf16; dx [T,B,C] bf16, d_maa [C]
+ *         (maa_dtype, NULL exactly when maa is), d_w_down / d_w_up in their own dtype codes,
+ *         d_bias in bias_dtype; sums over the tokens in fp32 in a fixed order.
+ * ---------------------------------------------------------------------- */
+int rwkv6_lora_down_fwd(const void* x, const void* maa, int maa_dtype, const void* w_down,
+                        int w_dtype, void* neck, int64_t T, int64_t B, int64_t C, int64_t E,
+                        int64_t R, void* stream);
+int rwkv6_lora_up_fwd(const void* x, const void* neck, const void* w_up, int w_dtype,
+                      const void* bias, int bias_dtype, void* const* out, int64_t T, int64_t B,
+                      int64_t C, int64_t E, int64_t R, void* stream);
+size_t rwkv6_lora_bwd_workspace_bytes(int64_t T, int64_t B, int64_t C, int64_t E, int64_t R);
+int rwkv6_lora_bwd(const void* x, const void* maa, int maa_dtype, const void* const* d_out,
+                   const void* neck, const void* w_down, const void* w_up, int w_dtype,
+                   const void* bias, int bias_dtype, void* dx, void* d_maa, void* d_w_down,
+                   int d_w_down_dtype, void* d_w_up, int d_w_up_dtype, void* d_bias,
+                   void* workspace, int64_t T, int64_t B, int64_t C, int64_t E, int64_t R,
+                   void* stream);
+
+/* ------------------------------------------------------------------------
  * Channel mix (RWKV6ChannelMix.forward, rwkv6_layer_specs.py:512-536), [T,B,C] bf16.
  *   mixed[e] = x + (shift(x) - x) * mix[e]    (:513-520), mix = mix_coeffs [2,C] in
  *              param_dtype; `mixed` is a host array of 2 device pointers, each [T,B,C]:

@@ -3,7 +3,11 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <atomic>
 #include <initializer_list>
+#include <mutex>
+
+#include "../../include/rwkv6_amd.h"
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
@@ -101,6 +105,50 @@ __device__ __forceinline__ void load_param8(const void* p, int dtype, int64_t of
     for (int s = 0; s < 8; ++s) f[s] = h ? hf[s] : __builtin_bit_cast(float, w[s]);
 }
 
+typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+// LDS transpose read (ds_read_b64_tr_b16): the 16 lanes of a row group supply four 8-byte chunks
+// of each of four rows, lane L receives column L of the four.
+
+__device__ __forceinline__ bf16x4 lds_tr16(const uint16_t* p) {
+    return __builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)p));
+}
+__device__ __forceinline__ bf16x8 cat_bf16x8(bf16x4 a, bf16x4 b) {
+    return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
+}
+// MFMA operand whose reduction runs over the rows of a row-major LDS tile: lane (q, L) receives
+// X[r0 + 8q + s][c0 + L], s = 0..7 (the slot order of a 16-byte row read).
+__device__ __forceinline__ bf16x8 lds_tr8(const uint16_t* X, int stride, int r0, int c0, int lane) {
+    const int L = lane & 15, q = lane >> 4;
+    const uint16_t* p = X + (r0 + 8 * q + (L >> 2)) * stride + c0 + 4 * (L & 3);
+    return cat_bf16x8(lds_tr16(p), lds_tr16(p + 4 * stride));
+}
+
+// Eight weights as loaded (bf16: one 16-byte piece; fp32: two), and as a bf16 piece.
+template <bool F32> struct WRaw { uint4 q[F32 ? 2 : 1]; };
+template <bool F32>
+__device__ __forceinline__ WRaw<F32> w_load(const void* w, int64_t off) {
+    WRaw<F32> r;
+    if constexpr (F32) {
+        const uint4* p = reinterpret_cast<const uint4*>(reinterpret_cast<const float*>(w) + off);
+        r.q[0] = p[0];
+        r.q[1] = p[1];
+    } else {
+        r.q[0] = *reinterpret_cast<const uint4*>(reinterpret_cast<const uint16_t*>(w) + off);
+    }
+    return r;
+}
+template <bool F32>
+__device__ __forceinline__ uint4 w_bf16(const WRaw<F32>& r) {
+    if constexpr (F32) {
+        return make_uint4(pk2(__uint_as_float(r.q[0].x), __uint_as_float(r.q[0].y)),
+                          pk2(__uint_as_float(r.q[0].z), __uint_as_float(r.q[0].w)),
+                          pk2(__uint_as_float(r.q[1].x), __uint_as_float(r.q[1].y)),
+                          pk2(__uint_as_float(r.q[1].z), __uint_as_float(r.q[1].w)));
+    } else {
+        return r.q[0];
+    }
+}
+
 // Lane exchanges without an address operand: DPP (a modifier of the consuming VALU op)
 // within rows of 16 lanes, ds_swizzle within 32 lanes; only the exchange across the two
 // 32-lane halves goes through ds_bpermute.
@@ -172,6 +220,44 @@ inline bool any_alias(std::initializer_list<Span> outs, std::initializer_list<Sp
     }
     return false;
 }
+
+namespace {
+constexpr int kMaxDevices = 64;
+
+// The device a call's kernels run on: the stream's, or the current one for the NULL stream.
+inline int stream_device(hipStream_t stream, int* dev, int* cur) {
+    if (hipGetDevice(cur) != hipSuccess) return RWKV6_ERR_LAUNCH;
+    *dev = *cur;
+    if (stream) {
+        hipDevice_t d = 0;
+        if (hipStreamGetDevice(stream, &d) != hipSuccess) return RWKV6_ERR_INVALID_ARG;
+        *dev = d;
+    }
+    return (*dev < 0 || *dev >= kMaxDevices) ? RWKV6_ERR_UNSUPPORTED : RWKV6_OK;
+}
+
+// Per-device set-up that is done once it has succeeded, with that device current: a failed
+// attempt is not cached, the next call tries again.  After the first success a call costs one
+// atomic load.  Set-up runs host API calls (attribute and symbol queries, no allocation); a
+// caller that captures the library's launches into a HIP graph makes one eager call on the
+// device first, so that none of it runs under capture.
+struct DeviceOnce {
+    std::mutex m;
+    std::atomic<bool> done{false};
+};
+template <class F>
+int device_once(DeviceOnce& slot, int dev, int cur, F&& body) {
+    if (slot.done.load(std::memory_order_acquire)) return RWKV6_OK;
+    std::lock_guard<std::mutex> lock(slot.m);
+    if (slot.done.load(std::memory_order_relaxed)) return RWKV6_OK;
+    hipError_t e = dev == cur ? hipSuccess : hipSetDevice(dev);
+    if (e == hipSuccess) e = body();
+    if (dev != cur) (void)hipSetDevice(cur);
+    if (e != hipSuccess) return RWKV6_ERR_LAUNCH;
+    slot.done.store(true, std::memory_order_release);
+    return RWKV6_OK;
+}
+}  // namespace
 
 // Second stage of every fixed-order reduction over token blocks: out[n] = sum_p part[p][n]
 // for fp32 partials part[P][Nn], written bf16 or fp32 (pdt); columns n >= split go to

@@ -66,6 +66,25 @@ __host__ __device__ __forceinline__ size_t lora_lds_bytes(int E, int R) {
     return (size_t)E * 64 * (R + 8) * 2;
 }
 
+// The same columns of W_up as the module holds it ([E*R][C], bf16 or fp32): rows = rank, read as
+// MFMA operands with the LDS transpose reads.
+#define LORA_NS 72                     // row stride (elements): 64 channels + 8
+template <bool F32>
+__device__ __forceinline__ void lora_stage_nat(uint16_t* sw, const void* wup, int ER, int64_t C, int64_t c0) {
+    for (int idx = threadIdx.x; idx < ER * 8; idx += LORA_THR)
+        *reinterpret_cast<uint4*>(sw + (idx >> 3) * LORA_NS + 8 * (idx & 7)) =
+            w_bf16<F32>(w_load<F32>(wup, (int64_t)(idx >> 3) * C + c0 + 8 * (idx & 7)));
+}
+// Operand rows tile_channel(tc, L), k = ranks r0 + 8q + s, of such a tile: the 16 channels of
+// tile tc are four 8-byte chunks 8 channels apart (tile_channel), which the transpose read
+// takes from any address.
+__device__ __forceinline__ bf16x8 lora_nat8(const uint16_t* sw, int r0, int tc, int lane) {
+    const int L = lane & 15, q = lane >> 4, j = L & 3;
+    const int col = tc < 2 ? 8 * j + 4 * tc : 32 + 8 * j + 4 * (tc - 2);
+    const uint16_t* p = sw + (r0 + 8 * q + (L >> 2)) * LORA_NS + col;
+    return cat_bf16x8(lds_tr16(p), lds_tr16(p + 4 * LORA_NS));
+}
+
 __device__ __forceinline__ void lora_stage(uint16_t* sw, const uint16_t* __restrict__ wut, int E,
                                            int64_t C, int R, int64_t c0) {
     const int rs = lds_rs(R), R8 = R / 8;
@@ -93,9 +112,10 @@ __device__ __forceinline__ void lora_stage(uint16_t* sw, const uint16_t* __restr
 // stores.  Loads and stores are unconditional: a token past the end works on the last token
 // and stores its values again (same values, same place).
 // KS = R / 32, or 0: from R at run time (ranks past the first 32 are then loaded in the stage).
-template <int E, bool LERP, int REP, int KS>
+// WL: the weights' layout, 0 = W_up^T [E,C,R] bf16, 1 and 2 = W_up [E,R,C] in bf16 and fp32.
+template <int E, bool LERP, int REP, int KS, int WL = 0>
 __global__ void __launch_bounds__(LORA_THR)
-rwkv6_lora_up_kernel(const uint16_t* __restrict__ neck, const uint16_t* __restrict__ wut,
+rwkv6_lora_up_kernel(const uint16_t* __restrict__ neck, const void* __restrict__ wut,
                      const void* __restrict__ bias, int pdt, const uint16_t* __restrict__ x,
                      OutPtrs<E> out, int64_t ors, int64_t N, int64_t B, int64_t C, int R,
                      int64_t per) {
@@ -112,7 +132,8 @@ rwkv6_lora_up_kernel(const uint16_t* __restrict__ neck, const uint16_t* __restri
     const int rw = lane >> 3, cg = lane & 7;
     const int64_t c0 = cb * 64, cl = c0 + 8 * cg;
     extern __shared__ __attribute__((aligned(16))) uint16_t lora_sm[];
-    lora_stage(lora_sm, wut, E, C, R, c0);
+    if constexpr (WL == 0) lora_stage(lora_sm, reinterpret_cast<const uint16_t*>(wut), E, C, R, c0);
+    else lora_stage_nat<WL == 2>(lora_sm, wut, E * R, C, c0);
     if (threadIdx.x < E * 8) {
         const int e = threadIdx.x >> 3, c8 = (threadIdx.x & 7) * 8;
         float bb[8];
@@ -163,8 +184,9 @@ rwkv6_lora_up_kernel(const uint16_t* __restrict__ neck, const uint16_t* __restri
                 const bf16x8 bq = __builtin_bit_cast(bf16x8, nkb[st % AH][ks]);
 #pragma unroll
                 for (int tcn = 0; tcn < 4; ++tcn)
-                    acc[tcn] = mfma32(ld_bf16x8(swe + tile_channel(tcn, L) * rs + 32 * ks + 8 * q), bq,
-                                      acc[tcn]);
+                    acc[tcn] = mfma32(WL == 0 ? ld_bf16x8(swe + tile_channel(tcn, L) * rs + 32 * ks + 8 * q)
+                                              : lora_nat8(lora_sm, e * R + 32 * ks, tcn, lane),
+                                      bq, acc[tcn]);
             }
             if (KS == 0) {
                 const uint16_t* nrow = neck + tok_m(g) * E * R + e * R + 8 * q;
@@ -661,6 +683,45 @@ int rwkv6_lora_bias_fwd(const void* neck, const void* w_up_t, const void* bias, 
                            lora_lds_bytes(LORA_NE, (int)R), s, (const uint16_t*)neck,
                            (const uint16_t*)w_up_t, bias, param_dtype, (const uint16_t*)nullptr, o,
                            (int64_t)LORA_NE * C, N, (int64_t)1, C, (int)R, up_per(N));
+    }
+    return launch_status();
+}
+
+int rwkv6_lora_up_fwd(const void* x, const void* neck, const void* w_up, int w_dtype,
+                      const void* bias, int bias_dtype, void* const* out, int64_t T, int64_t B,
+                      int64_t C, int64_t E, int64_t R, void* stream) {
+    if (T < 0 || B < 1 || E < 1) return RWKV6_ERR_INVALID_ARG;
+    const bool lerp = E == LORA_NE;
+    if (lerp ? R != 32 : (E != 1 || R != 64)) return RWKV6_ERR_UNSUPPORTED;
+    int st = lora_check((int)E, T * B, C, R, bias_dtype);
+    if (st) return st;
+    if (w_dtype != RWKV6_F32 && w_dtype != RWKV6_BF16) return RWKV6_ERR_INVALID_ARG;
+    if (T == 0) return RWKV6_OK;
+    if (!neck || !w_up || !bias || !out || lerp != (x != nullptr)) return RWKV6_ERR_INVALID_ARG;
+    if (!al16(x) || !al16(neck) || !al16(w_up) || !al16(bias)) return RWKV6_ERR_ALIGNMENT;
+    OutPtrs<LORA_NE> o{};
+    if ((st = lerp ? gather<OutPtrs<LORA_NE>, LORA_NE>((const void* const*)out, o)
+                   : gather<OutPtrs<LORA_NE>, 1>((const void* const*)out, o)))
+        return st;
+    const int64_t N = T * B;
+    const size_t act = (size_t)(N * C) * 2;
+    if (any_alias({{o.p[0], act}, {o.p[1], act}, {o.p[2], act}, {o.p[3], act}, {o.p[4], act}},
+                  {{x, act}, {neck, (size_t)(N * E * R) * 2}, {w_up, (size_t)(E * C * R) * param_bytes(w_dtype)},
+                   {bias, (size_t)(E * C) * param_bytes(bias_dtype)}}))
+        return RWKV6_ERR_INVALID_ARG;
+    hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+    const size_t lds = (size_t)E * R * LORA_NS * 2;
+    const bool f32 = w_dtype == RWKV6_F32;
+    if (lerp) {
+        auto kern = f32 ? rwkv6_lora_up_kernel<LORA_NE, true, 1, 1, 2> : rwkv6_lora_up_kernel<LORA_NE, true, 1, 1, 1>;
+        hipLaunchKernelGGL(kern, up_grid(N, C), dim3(LORA_THR), lds, s, (const uint16_t*)neck, w_up, bias,
+                           bias_dtype, (const uint16_t*)x, o, C, N, B, C, (int)R, up_per(N));
+    } else {
+        OutPtrs<1> o1;
+        o1.p[0] = o.p[0];
+        auto kern = f32 ? rwkv6_lora_up_kernel<1, false, 4, 2, 2> : rwkv6_lora_up_kernel<1, false, 4, 2, 1>;
+        hipLaunchKernelGGL(kern, up_grid(N, C, 4), dim3(LORA_THR), lds, s, (const uint16_t*)neck, w_up, bias,
+                           bias_dtype, (const uint16_t*)nullptr, o1, C, N, (int64_t)1, C, (int)R, up_per(N, 4));
     }
     return launch_status();
 }

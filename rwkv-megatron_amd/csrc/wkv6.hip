@@ -47,8 +47,6 @@
 // accumulators by the very bf16 Rm, Km the products used, so it does (single bf16 operands,
 // no hi + lo split).
 #include <algorithm>
-#include <atomic>
-#include <mutex>
 
 #include "common.h"
 #include "../../include/rwkv6_amd.h"
@@ -72,7 +70,6 @@
 #define FLOOR_FF 21807.29f    // e^{-W_MIN - 0.01}: Fm Fk above it marks a floored token
 
 typedef uint16_t tile_t[CL][TS];
-typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 
 // ---------------------------------------------------------------------------
 // operand fragments
@@ -2621,42 +2618,6 @@ size_t rwkv6_wkv_workspace_bytes(int64_t B, int64_t H, int64_t T, int64_t K, int
 }  // extern "C"
 
 namespace {
-
-constexpr int kMaxDevices = 64;
-
-// The device a call's kernels run on: the stream's, or the current one for the NULL stream.
-int stream_device(hipStream_t stream, int* dev, int* cur) {
-    if (hipGetDevice(cur) != hipSuccess) return RWKV6_ERR_LAUNCH;
-    *dev = *cur;
-    if (stream) {
-        hipDevice_t d = 0;
-        if (hipStreamGetDevice(stream, &d) != hipSuccess) return RWKV6_ERR_INVALID_ARG;
-        *dev = d;
-    }
-    return (*dev < 0 || *dev >= kMaxDevices) ? RWKV6_ERR_UNSUPPORTED : RWKV6_OK;
-}
-
-// Per-device set-up that is done once it has succeeded, with that device current: a failed
-// attempt is not cached, the next call tries again.  After the first success a call costs one
-// atomic load.  Set-up runs host API calls (attribute and symbol queries, no allocation); a
-// caller that captures the library's launches into a HIP graph makes one eager call on the
-// device first, so that none of it runs under capture.
-struct DeviceOnce {
-    std::mutex m;
-    std::atomic<bool> done{false};
-};
-template <class F>
-int device_once(DeviceOnce& slot, int dev, int cur, F&& body) {
-    if (slot.done.load(std::memory_order_acquire)) return RWKV6_OK;
-    std::lock_guard<std::mutex> lock(slot.m);
-    if (slot.done.load(std::memory_order_relaxed)) return RWKV6_OK;
-    hipError_t e = dev == cur ? hipSuccess : hipSetDevice(dev);
-    if (e == hipSuccess) e = body();
-    if (dev != cur) (void)hipSetDevice(cur);
-    if (e != hipSuccess) return RWKV6_ERR_LAUNCH;
-    slot.done.store(true, std::memory_order_release);
-    return RWKV6_OK;
-}
 
 // The dynamic-LDS limit of every kernel here that takes more than 64 KB, raised once per
 // device instead of on every call.

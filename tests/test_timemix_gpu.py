@@ -332,3 +332,57 @@ def test_empty_inputs_zero_parameter_gradients(pkg):
     for name, t in (("col_sum", out), ("d_maa", d_maa), ("d_mix", d_mix), ("dgamma", dgamma),
                     ("dbeta", dbeta), ("d_bias", d_bias)):
         assert torch.equal(t, torch.zeros_like(t)), name
+
+
+def _bottleneck_case(form, T, B, C, wdt, udt, pdt):
+    """Leaves and output gradients of one bottleneck call; x non-contiguous for odd T."""
+    g = torch.Generator().manual_seed(1000 * T + 10 * B + C)
+    E, R = (5, 32) if form == "mix" else (1, 64)
+    x = _bf(torch.randn(B, T, C, generator=g)).transpose(0, 1) if T % 2 else _bf(torch.randn(T, B, C, generator=g))
+    wd = _bf(torch.randn(C, E, R, generator=g) * 0.5 * C ** -0.5).to(wdt)
+    wu = _bf(torch.randn(E, R, C, generator=g) * 0.05).to(udt)
+    bias = torch.rand(E, C, generator=g).to(pdt)
+    maa = torch.rand(C, generator=g).to(pdt)
+    dy = [_bf(torch.randn(T, B, C, generator=g)).to(DEV) for _ in range(E)]
+    return [t.to(DEV) for t in (x, maa, wd, wu, bias)], dy
+
+
+def _bottleneck_run(pkg, form, leaves, dy):
+    leaves = [t.detach().requires_grad_(True) for t in leaves]
+    x, maa, wd, wu, bias = leaves
+    out = (pkg.timemix.token_shift_mix(*leaves) if form == "mix"
+           else (pkg.timemix.decay_lora(x, wd, wu, bias),))
+    wrt = leaves if form == "mix" else [x, wd, wu, bias]
+    return [t.detach() for t in out] + list(torch.autograd.grad(out, wrt, dy))
+
+
+# Tokens at the edges of the kernels' tiles (64 rows; the token-shift gradient kernel steps 63 of
+# one batch column, the others 64 rows of all), one to three channel blocks, several ranges, and
+# every mix of parameter dtypes.  Both paths round the same operands to bf16 and sum in fp32; the
+# general path rounds its neck and three intermediate gradients once more (2^-9 each, 2^-8 over
+# the worst sum of them), the outputs of either are rounded once: 1.6e-2 relative L2 is four
+# times the sum of those.
+@pytest.mark.parametrize("form", ["mix", "decay"])
+@pytest.mark.parametrize("T,B,C,wdt,udt,pdt", [
+    (0, 2, 64, torch.bfloat16, torch.bfloat16, torch.bfloat16),
+    (1, 1, 64, torch.bfloat16, torch.bfloat16, torch.float32),
+    (1, 65, 64, torch.float32, torch.float32, torch.float32),
+    (2, 1, 128, torch.float32, torch.bfloat16, torch.bfloat16),
+    (63, 2, 64, torch.bfloat16, torch.bfloat16, torch.bfloat16),
+    (64, 1, 192, torch.float32, torch.float32, torch.bfloat16),
+    (65, 1, 64, torch.bfloat16, torch.float32, torch.float32),
+    (127, 3, 64, torch.float32, torch.float32, torch.float32),
+    (128, 1, 64, torch.float16, torch.bfloat16, torch.float16),
+    (1009, 2, 512, torch.bfloat16, torch.bfloat16, torch.bfloat16)])
+def test_bottleneck_kernels_match_the_general_path(pkg, monkeypatch, form, T, B, C, wdt, udt, pdt):
+    leaves, dy = _bottleneck_case(form, T, B, C, wdt, udt, pdt)
+    got = _bottleneck_run(pkg, form, leaves, dy)
+    again = _bottleneck_run(pkg, form, leaves, dy)
+    monkeypatch.setattr(pkg.timemix, "_FUSED", set())
+    ref = _bottleneck_run(pkg, form, leaves, dy)
+    torch.cuda.synchronize()
+    for i, (a, b, c) in enumerate(zip(got, again, ref)):
+        assert a.dtype == c.dtype and a.shape == c.shape and torch.equal(a, b)
+        if a.numel():
+            err = float((a.double() - c.double()).norm() / c.double().norm().clamp_min(1e-20))
+            assert err <= 1.6e-2 or float(c.double().abs().max()) == 0.0 == float(a.double().abs().max()), (i, err)
