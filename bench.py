@@ -249,30 +249,25 @@ def config1_bench(pkg, gpu_steps, with_cpu):
     return out
 
 
-def bwd_walk_segments(BH, T):
-    """Segments per sequence of the library's reverse walk (wkv6_bwd_loop), 0 when the backward
-    runs chunk-parallel: the rule of bwd_walk_segments() in csrc/wkv6.hip (walk_segments() with
-    a 256-workgroup target; the walk when it is one segment or the segments fill 7/8 of it)."""
-    NT = -(-T // 64)
-    if NT <= 0:
-        return 1
-    P = min(max(1, 256 // BH), max(1, NT // 8))
-    NC = -(-NT // P)
-    P = -(-NT // NC)
-    return P if P == 1 or 8 * BH * P >= 7 * 256 else 0
+def bwd_plan(BH, T):
+    """The library's plan for the backward of BH sequences (rwkv6_wkv_plan): segments a sequence,
+    negative when they form their own starting state gradients, 0 for chunk-parallel."""
+    return importlib.import_module("rwkv-megatron_amd")._lib.load().rwkv6_wkv_plan(BH, 1, T, 1)
 
 
 def bwd_kernel(BH, T):
-    return "wkv6_bwd_loop" if bwd_walk_segments(BH, T) else "wkv6_bwd_chunk_grads"
+    return "wkv6_bwd_loop" if bwd_plan(BH, T) else "wkv6_bwd_chunk_grads"
 
 
 def bwd_path(BH, T):
-    P = bwd_walk_segments(BH, T)
+    P = bwd_plan(BH, T)
     if P == 1:
         return "reverse walk (wkv6_bwd_loop)"
     if P > 1:
         return (f"segmented reverse walk ({P} segments: wkv6_bwd_pieces, wkv6_bwd_fold, "
                 "wkv6_bwd_loop)")
+    if P < 0:
+        return f"segmented reverse walk ({-P} segments that form their own starts: wkv6_bwd_loop)"
     return "chunk-parallel (wkv6_bwd_chunk_dstate, wkv6_state_scan_bwd, wkv6_bwd_chunk_grads)"
 
 

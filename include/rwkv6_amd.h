@@ -278,6 +278,10 @@ int rwkv6_wkv_fwd_noalloc(const void* r, const void* k, const void* v, const voi
  *   bwd: 0 chunk-local dstates (chunk-parallel form only), 1 the reverse dstate walk or
  *        the dstate scan, 2 chunk gradients, 3 du reduction
  * ---------------------------------------------------------------------- */
+/* How a shape runs (for labels and tests): P > 0: P segments a sequence, started by a pre-pass
+ * when P > 1; -P: P segments that form their own start states; 0: the chunk-parallel backward
+ * (or T = 0, or a bad shape). */
+int rwkv6_wkv_plan(int64_t B, int64_t H, int64_t T, int for_bwd);
 int rwkv6_wkv_fwd_ex(const void* r, const void* k, const void* v, const void* w, const void* u,
                      int u_dtype, const float* h0, void* o, float* hT, void* saved,
                      void* workspace, int64_t B, int64_t H, int64_t T, int64_t K, int64_t V,

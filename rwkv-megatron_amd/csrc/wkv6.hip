@@ -5,7 +5,9 @@
 //   o_t = s * r_t^T (S_{t-1} + diag(u) k_t v_t^T),   S_t = diag(exp(w_t)) S_{t-1} + k_t v_t^T.
 //
 // Decomposition (all deterministic):
-//   wkv6_fwd_pieces  only when B*H gives fewer than 256 workgroups: per (b,h, piece of segments
+//   Sequences that leave CUs idle are cut into segments (walk_plan); a segment's start state
+//   comes from a pre-pass, or from the walk itself for short sequences (its PRE form).
+//   wkv6_fwd_pieces  the pre-pass: per (b,h, piece of segments
 //                    0..P-2), the piece's end state from a zero start and its total decay
 //                    (k, v, w read once more)
 //   wkv6_fwd_fold    chains the pieces from h0 into each segment's start state
@@ -19,8 +21,8 @@
 //   wkv6_bwd_loop    per (b,h, segment): the reverse walk, all gradients of each chunk with
 //                    dS_out(c-1) = e^{G_63} dS_out(c) + s sum_t (r_t e^{G_{t-1}}) dO_t^T  [MFMA]
 //                    carried in registers; dh0 and the du partials
-//   chunk-parallel backward, when even the segments cannot fill the device (few, short
-//   sequences):
+//   chunk-parallel backward, where the plan's model has it ahead of the walk (few sequences,
+//   few chunks):
 //     wkv6_bwd_chunk_dstate  per (b,h, chunk): dS_loc and the chunk decay                [MFMA]
 //     wkv6_state_scan_bwd    per (b,h, element): dS_out(c-1) = e^{G_63(c)} dS_out(c) + dS_loc(c)
 //     wkv6_bwd_chunk_grads   per (b,h, chunk): dr, dk, dv, dw, du partials               [MFMA]
@@ -260,10 +262,6 @@ __host__ __device__ constexpr int pair_index(int I, int J) { return I * (I - 1) 
 #ifndef WALK_TARGET_ITEMS
 #define WALK_TARGET_ITEMS 256   // workgroups a forward should offer (one per CU of an MI355X)
 #endif
-#define WALK_MIN_CHUNKS 8       // shortest segment worth a pre-pass
-#ifndef DSTATE_TARGET_ITEMS
-#define DSTATE_TARGET_ITEMS 256 // the same for the backward's walk
-#endif
 #ifndef WALK_WPE
 #define WALK_WPE 2              // waves per SIMD the walk is compiled for (1 block of 8 waves / CU)
 #endif
@@ -356,18 +354,6 @@ __device__ __forceinline__ void walk_scan2(WalkSmem& sm, const float* loc, int t
     }
 }
 
-// Segments per sequence (shared by the workspace query and the launch): as many (b,h, segment)
-// workgroups as fit `target` (one walk per CU) without a second round, no segment shorter
-// than WALK_MIN_CHUNKS.  (Rounding up instead, e.g. 3 segments for 96 sequences, put the 288
-// walks into two rounds: 30 % slower at B*H = 96, T = 4096.)
-inline int walk_segments(int64_t BH, int64_t NT, int64_t target = WALK_TARGET_ITEMS) {
-    if (NT <= 0) return 1;
-    int64_t P = target / BH > 1 ? target / BH : 1;
-    P = std::min<int64_t>(P, std::max<int64_t>(1, NT / WALK_MIN_CHUNKS));
-    const int64_t NC = (NT + P - 1) / P;               // chunks per segment
-    return (int)((NT + NC - 1) / NC);                   // no empty segment
-}
-
 // Pieces of the forward pre-pass (wkv6_fwd_pieces): each of the P-1 earlier segments of a
 // sequence is cut into `sub` pieces of at most `ncs` chunks, `sub` the nearest integer to
 // PIECE_TARGET / (B*H*(P-1)) (about one piece per CU: with most CUs busy the pre-pass is bound
@@ -391,14 +377,57 @@ inline Pieces prepass_pieces(int64_t BH, int64_t NT, int P, int64_t max_pieces) 
     return {(int)((NC + ncs - 1) / ncs), (int)ncs};      // no empty piece, sub only shrinks
 }
 
-// The backward walks each sequence in one workgroup (wkv6_bwd_loop) when there is one segment;
-// with fewer sequences, each is cut into segments like the forward's as long as the (b,h,
-// segment) workgroups fill at least 7/8 of the device (a segment walks at ~6 us a chunk
-// whatever the occupancy).  Otherwise (few, short segments) the state gradients run
-// chunk-parallel.  Returns the segment count of the walk, or 0 for the chunk-parallel form.
-inline int bwd_walk_segments(int64_t BH, int64_t NT) {
-    const int P = walk_segments(BH, NT, DSTATE_TARGET_ITEMS);
-    return (P == 1 || 8 * BH * P >= 7 * DSTATE_TARGET_ITEMS) ? P : 0;
+// How a walk is cut (shared by the workspace query and the launch): P segments a sequence, one
+// (b,h, segment) walk per CU in one round (256 workgroups; a second round cost 30 % at B*H = 96,
+// T = 4096), and where segments start from: `pre`: each forms its start state itself from the
+// chunks before it (backward: after it), else (P > 1) a pre-pass of pieces and a fold do.  P = 0
+// (backward only): the chunk-parallel form.
+// The plan is the fastest by a model in microseconds, fitted to kernels timed on MI355X over
+// B*H = 8..128 and 2..128 chunks (back to back, without launch gaps):
+//   a walk                    chunk us for each chunk of the longest segment
+//   pre                       head + step us for each 128 tokens of the longest prefix
+//   pre-pass (two launches)   9.5 + 0.4 a piece of the sequence + 1.6 for each 128 tokens of a piece
+//   chunk-parallel (four)     12.8 + 0.029 a (b,h, chunk), over what a walk needs besides its chunks
+// (a launch beyond the walk's own is counted as 2 us).  E.g., one segment -> plan: forward of 16
+// sequences of 8 chunks 22.5 -> 15.0 us (pre, 8 segments), of 32 sequences of 32 chunks 34.8 ->
+// 28.3 (pre-pass, 8 segments of 4 chunks instead of 4 of 8); backward of the same 43.9 -> 20.4
+// (pre; chunk-parallel 18.9 with two launches more) and 57.2 -> 42.1, of 8 sequences of 13 chunks
+// 66.5 -> 19.9 (chunk-parallel).
+struct WalkPlan {
+    int P;
+    bool pre;
+};
+struct WalkModel {
+    double chunk, head, step;
+};
+constexpr WalkModel FWD_MODEL{2.25, 0.7, 1.6}, BWD_MODEL{4.62, 2.0, 1.8};
+inline WalkPlan walk_plan(int64_t BH, int64_t NT, const WalkModel& m, double* cost) {
+    WalkPlan best{1, false};
+    *cost = NT * m.chunk;
+    if (BH > WALK_TARGET_ITEMS / 2) return best;
+    // segment lengths from the shortest that one round takes, in steps of a quarter (the plan of
+    // a call must cost little: a handful of candidates)
+    const int nt = (int)NT, pmax = WALK_TARGET_ITEMS / (int)BH;
+    for (int NC = (nt + pmax - 1) / pmax; NC < nt; NC += std::max(1, NC / 4)) {
+        const int P = (nt + NC - 1) / NC;
+        const Pieces pc = prepass_pieces(BH, NT, P, PIECE_TARGET);
+        const double pre = m.head + ((P - 1) * NC + 1) / 2 * m.step + NC * m.chunk;
+        const double pieces = 9.5 + 0.4 * ((P - 1) * pc.sub) + (pc.ncs + 1) / 2 * 1.6 + NC * m.chunk;
+        if (std::min(pre, pieces) < *cost) {
+            *cost = std::min(pre, pieces);
+            best = {P, pre <= pieces};
+        }
+    }
+    return best;
+}
+inline WalkPlan fwd_walk_plan(int64_t BH, int64_t NT) {
+    double cost;
+    return walk_plan(BH, NT, FWD_MODEL, &cost);
+}
+inline WalkPlan bwd_walk_plan(int64_t BH, int64_t NT) {
+    double cost;
+    const WalkPlan p = walk_plan(BH, NT, BWD_MODEL, &cost);
+    return NT < 2 || cost <= 12.8 + 0.029 * (double)(BH * NT) ? p : WalkPlan{0, false};
 }
 
 struct WalkPrefetch {
@@ -692,105 +721,9 @@ __device__ __forceinline__ void fwd_walk_chunks(
 
 }
 
-// Output walk over segment blockIdx.x % P of sequence blockIdx.x / P.  Segment 0 starts from
-// h0 (or zero), segment p >= 1 from Sstart[b,h][p-1] (wkv6_fwd_fold).
-// SEQ: r, k, v and the pre-activation decay are sequence-first; o is always head-first.
-template <bool SEQ>
-__global__ void __launch_bounds__(NTHR_W) __attribute__((amdgpu_waves_per_eu(WALK_WPE)))
-wkv6_fwd_walk(const uint16_t* __restrict__ r, const uint16_t* __restrict__ k,
-              const uint16_t* __restrict__ v, const uint16_t* __restrict__ w,
-              const void* __restrict__ u, int u_dtype, const float* __restrict__ h0,
-              uint16_t* __restrict__ o, uint16_t* __restrict__ Hs, float* __restrict__ hT,
-              const float* __restrict__ Sstart, float scale, int B, int H, int T, int NT, int P) {
-    extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
-    WalkSmem& sm = *reinterpret_cast<WalkSmem*>(smem_raw);
-    const int bh = blockIdx.x / P, seg = blockIdx.x - bh * P, h = bh % H;
-    const int NC = (NT + P - 1) / P;
-    const int c_begin = seg * NC, c_end = min(NT, c_begin + NC);
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    // waves 0-3 take token blocks 0,0,1,1 and waves 4-7 blocks 3,3,2,2: with waves dealt
-    // round-robin to the 4 SIMDs, each SIMD gets blocks {0,3} or {1,2}, whose cross-block
-    // work (W products each) sums to the same 3
-    const int W = wv < 4 ? (wv >> 1) : 5 - (wv >> 1), hh = wv & 1;
-    const int lr = lane & 15, lq = lane >> 4;
-    const size_t sbase = (size_t)bh * KD * KD;
-
-    WalkPrefetch nx;
-    if (c_begin < c_end) walk_issue<SEQ>(nx, r, k, v, w, bh, c_begin, c_begin, B, H, T);
-
-    // ---- starting state ----
-    f32x4 acc[2];
-    {
-        const float* s0 = seg > 0 ? Sstart + ((size_t)bh * (P - 1) + seg - 1) * KD * KD
-                                  : (h0 ? h0 + sbase : nullptr);
-        // one branch around all eight loads (a conditional per element came out ~1 % slower
-        // over the whole walk: the register assignment of the loop differed)
-        if (s0) {
-#pragma unroll
-            for (int tp = 0; tp < 2; ++tp) {
-                const float4 x = *reinterpret_cast<const float4*>(
-                    s0 + (16 * W + lr) * KD + 32 * hh + 16 * tp + 4 * lq);
-                acc[tp][0] = x.x; acc[tp][1] = x.y; acc[tp][2] = x.z; acc[tp][3] = x.w;
-            }
-        } else {
-#pragma unroll
-            for (int tp = 0; tp < 2; ++tp)
-#pragma unroll
-                for (int rr = 0; rr < 4; ++rr) acc[tp][rr] = 0.f;
-        }
-        if (threadIdx.x < KD) sm.uh[threadIdx.x] = load_u(u, u_dtype, h * KD + threadIdx.x);
-        if (threadIdx.x < GSG) sm.G[threadIdx.x] = 0.f;       // G before the chunk: 0
-        __syncthreads();
-    }
-
-    switch (__builtin_amdgcn_readfirstlane(wv >> 1)) {
-    case 0:
-        fwd_walk_chunks<SEQ, 0>(sm, r, k, v, w, o, Hs, scale, B, H, T, NT, bh, c_begin, c_end, hh, nx, acc);
-        break;
-    case 1:
-        fwd_walk_chunks<SEQ, 1>(sm, r, k, v, w, o, Hs, scale, B, H, T, NT, bh, c_begin, c_end, hh, nx, acc);
-        break;
-    case 2:
-        fwd_walk_chunks<SEQ, 2>(sm, r, k, v, w, o, Hs, scale, B, H, T, NT, bh, c_begin, c_end, hh, nx, acc);
-        break;
-    default:
-        fwd_walk_chunks<SEQ, 3>(sm, r, k, v, w, o, Hs, scale, B, H, T, NT, bh, c_begin, c_end, hh, nx, acc);
-        break;
-    }
-
-    // ---- end of the sequence: the final state ----
-    if (seg == P - 1) {
-#pragma unroll
-        for (int tp = 0; tp < 2; ++tp) {
-            const size_t e = (size_t)(16 * W + lr) * KD + 32 * hh + 16 * tp + 4 * lq;
-            *reinterpret_cast<uint2*>(Hs + (size_t)bh * (NT + 1) * KD * KD + (size_t)NT * KD * KD + e) =
-                make_uint2(pk2(acc[tp][0], acc[tp][1]), pk2(acc[tp][2], acc[tp][3]));
-            if (hT)
-                *reinterpret_cast<float4*>(hT + sbase + e) =
-                    make_float4(acc[tp][0], acc[tp][1], acc[tp][2], acc[tp][3]);
-        }
-    }
-}
-
 // ---------------------------------------------------------------------------
-// forward pre-pass: the end states of runs of chunks ("pieces")
+// states over runs of chunks (the pre-pass pieces, and the walks' own prefixes)
 // ---------------------------------------------------------------------------
-// Segment p of the output walk starts from the state entering its first chunk.  Each of the
-// segments 0..P-2 is cut into SUB pieces of at most NCS chunks; one workgroup per (b,h, piece)
-// walks its chunks from a zero state, two chunks (PSPAN = 128 tokens) per step,
-//   S = diag(e^{G_end}) S + sum_tau (k_tau e^{G_end - G_tau}) v_tau^T        [MFMA]
-// with G the cumulative log-decay over the step, and writes the piece's end state S_q (fp32
-// [64][64]) and total log2-decay A_q ([64]).  Only k, v and w are read.  Per step, thread
-// (part, i) scans the log-decay of channel i over the tokens 16 part .. 16 part + 15 and forms
-// those tokens' k e^{G_end - G} itself, written channel-major (two 16-byte stores) as the
-// MFMA's A operand: no cumulative-decay tile.  The raw tiles are double-buffered, so a step
-// takes two barriers (piece_steps: the next step's scan runs beside this step's state
-// update; four before, 78.4 -> 76.8 us at config 5).  The exponents G_end - G_tau are never
-// positive, whatever the step's length, so the end state needs none of the walk's 64-token
-// references; 128-token steps halve the barriers per token (86.7 against 89.2 us at config 5
-// with one 64-token chunk per step; loads two steps ahead measured no faster, and a plain
-// read stream of the same shape, one workgroup per CU, takes 59 us).  With 132 KB of LDS a
-// piece takes a CU to itself; prepass_pieces caps the pieces at one per CU.
 #define PSPAN (2 * CL)     // tokens per step of the pre-pass pieces
 #define PETS (PSPAN + 8)   // row stride of the channel-major operand tile (elements)
 typedef uint16_t ptile_t[PSPAN][TS];
@@ -803,6 +736,7 @@ struct PieceSmem {
                                       // forward, r e^{G_{t-1}} backward
 };
 static_assert(sizeof(PieceSmem) <= 160 * 1024, "piece block LDS");
+#define WALK_PRE_LDS std::max(sizeof(WalkSmem), sizeof(PieceSmem))
 
 // A step of a pre-pass piece is three parts on raw tiles in LDS (nvalid tokens; the rows past
 // them zeroed), spread over two barriers so that the decay scan of the next step shares the
@@ -906,6 +840,7 @@ __device__ __forceinline__ void piece_store(PieceSmem& sm, int b, PieceLoads& f,
 // state update of step s and the scan of step s + 1.  `issue(m)` loads step m into nx and
 // `nvalid(m)` counts its tokens.  Past the last step the indices stay on it (unconditional
 // loads and stores; the extra scan is never used).
+#define PIECE_BARRIERS(nsteps) (2 + 2 * (nsteps))      // barriers of piece_steps
 template <bool SEQ, bool BWD, class Issue, class Nvalid>
 __device__ __forceinline__ void piece_steps(PieceSmem& sm, PieceLoads& nx, int nsteps, Issue issue,
                                             Nvalid nvalid, f32x4* acc, float& gsum) {
@@ -929,6 +864,162 @@ __device__ __forceinline__ void piece_steps(PieceSmem& sm, PieceLoads& nx, int n
     }
 }
 
+// The state entering chunk c_end of a sequence, from h0 (or zero), in the walk's layout: lane
+// (lq, lr) of wave (W, hh) gets S[16W + lr][32hh + 16tp + 4lq + rr].  All of the walk's 512
+// threads; LDS is free again after it.
+#define PST 68             // row stride (floats) of the fp32 state handed through LDS
+template <bool SEQ>
+__device__ __forceinline__ void fwd_prefix(unsigned char* smem, const uint16_t* __restrict__ k,
+                                           const uint16_t* __restrict__ v,
+                                           const uint16_t* __restrict__ w,
+                                           const float* __restrict__ h0, int bh, int c_end, int B,
+                                           int H, int T, int W, int hh, f32x4* acc) {
+    PieceSmem& ps = *reinterpret_cast<PieceSmem*>(smem);
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, lr = lane & 15, lq = lane >> 4;
+    const int row = threadIdx.x >> 3, c8 = (threadIdx.x & 7) * 8;
+    const int PW = wv >> 1, t_end = c_end * CL, nsteps = (c_end + 1) / 2;   // c_end chunks, all whole
+    const size_t rs = tok_rs<SEQ>(B, H);
+    PieceLoads nx;
+    auto issue = [&](int m) {
+        const int t0 = 2 * m * CL, nv = min(PSPAN, t_end - t0);
+        const size_t base = tok_base<SEQ>(bh, t0, B, H, T);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const size_t off = base + (size_t)min(row + 64 * h, nv - 1) * rs + c8;
+            nx.x[h] = *reinterpret_cast<const uint4*>(k + off);
+            nx.y[h] = *reinterpret_cast<const uint4*>(v + off);
+            nx.w[h] = *reinterpret_cast<const uint4*>(w + off);
+        }
+    };
+    auto nvalid = [&](int m) { return min(PSPAN, t_end - 2 * m * CL); };
+    f32x4 st[2] = {};
+    if (h0) {
+#pragma unroll
+        for (int tp = 0; tp < 2; ++tp)
+#pragma unroll
+            for (int rr = 0; rr < 4; ++rr) st[tp][rr] = h0[(16 * PW + 4 * lq + rr) * KD + 32 * hh + 16 * tp + lr];
+    }
+    float gsum = 0.f;
+    piece_steps<SEQ, false>(ps, nx, nsteps, issue, nvalid, st, gsum);
+    float* x = reinterpret_cast<float*>(smem);
+#pragma unroll
+    for (int tp = 0; tp < 2; ++tp)
+#pragma unroll
+        for (int rr = 0; rr < 4; ++rr) x[(16 * PW + 4 * lq + rr) * PST + 32 * hh + 16 * tp + lr] = st[tp][rr];
+    __syncthreads();
+#pragma unroll
+    for (int tp = 0; tp < 2; ++tp)
+        acc[tp] = *reinterpret_cast<const f32x4*>(x + (16 * W + lr) * PST + 32 * hh + 16 * tp + 4 * lq);
+    __syncthreads();
+}
+
+// Output walk over segment blockIdx.x % P of sequence blockIdx.x / P.  Segment 0 starts from
+// h0 (or zero), segment p >= 1 from Sstart[b,h][p-1] (wkv6_fwd_fold).
+// SEQ: r, k, v and the pre-activation decay are sequence-first; o is always head-first.
+// PRE: segment p >= 1 forms its start state itself, from h0 and the chunks before it (piece
+// steps of 128 tokens), instead of reading it from a pre-pass: one launch instead of three for
+// sequences short enough that re-reading the prefix costs less (walk_plan).
+template <bool SEQ, bool PRE>
+__global__ void __launch_bounds__(NTHR_W) __attribute__((amdgpu_waves_per_eu(WALK_WPE)))
+wkv6_fwd_walk(const uint16_t* __restrict__ r, const uint16_t* __restrict__ k,
+              const uint16_t* __restrict__ v, const uint16_t* __restrict__ w,
+              const void* __restrict__ u, int u_dtype, const float* __restrict__ h0,
+              uint16_t* __restrict__ o, uint16_t* __restrict__ Hs, float* __restrict__ hT,
+              const float* __restrict__ Sstart, float scale, int B, int H, int T, int NT, int P) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+    WalkSmem& sm = *reinterpret_cast<WalkSmem*>(smem_raw);
+    const int bh = blockIdx.x / P, seg = blockIdx.x - bh * P, h = bh % H;
+    const int NC = (NT + P - 1) / P;
+    const int c_begin = seg * NC, c_end = min(NT, c_begin + NC);
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    // waves 0-3 take token blocks 0,0,1,1 and waves 4-7 blocks 3,3,2,2: with waves dealt
+    // round-robin to the 4 SIMDs, each SIMD gets blocks {0,3} or {1,2}, whose cross-block
+    // work (W products each) sums to the same 3
+    const int W = wv < 4 ? (wv >> 1) : 5 - (wv >> 1), hh = wv & 1;
+    const int lr = lane & 15, lq = lane >> 4;
+    const size_t sbase = (size_t)bh * KD * KD;
+
+    f32x4 acc[2];
+    if constexpr (PRE) {
+        if (seg > 0) fwd_prefix<SEQ>(smem_raw, k, v, w, h0 ? h0 + sbase : nullptr, bh, c_begin, B, H, T, W, hh, acc);
+    }
+    WalkPrefetch nx;
+    if (c_begin < c_end) walk_issue<SEQ>(nx, r, k, v, w, bh, c_begin, c_begin, B, H, T);
+
+    // ---- starting state ----
+    if (!PRE || seg == 0) {
+        const float* s0 = seg > 0 ? Sstart + ((size_t)bh * (P - 1) + seg - 1) * KD * KD
+                                  : (h0 ? h0 + sbase : nullptr);
+        // one branch around all eight loads (a conditional per element came out ~1 % slower
+        // over the whole walk: the register assignment of the loop differed)
+        if (s0) {
+#pragma unroll
+            for (int tp = 0; tp < 2; ++tp) {
+                const float4 x = *reinterpret_cast<const float4*>(
+                    s0 + (16 * W + lr) * KD + 32 * hh + 16 * tp + 4 * lq);
+                acc[tp][0] = x.x; acc[tp][1] = x.y; acc[tp][2] = x.z; acc[tp][3] = x.w;
+            }
+        } else {
+#pragma unroll
+            for (int tp = 0; tp < 2; ++tp)
+#pragma unroll
+                for (int rr = 0; rr < 4; ++rr) acc[tp][rr] = 0.f;
+        }
+    }
+    {
+        if (threadIdx.x < KD) sm.uh[threadIdx.x] = load_u(u, u_dtype, h * KD + threadIdx.x);
+        if (threadIdx.x < GSG) sm.G[threadIdx.x] = 0.f;       // G before the chunk: 0
+        __syncthreads();
+    }
+
+    switch (__builtin_amdgcn_readfirstlane(wv >> 1)) {
+    case 0:
+        fwd_walk_chunks<SEQ, 0>(sm, r, k, v, w, o, Hs, scale, B, H, T, NT, bh, c_begin, c_end, hh, nx, acc);
+        break;
+    case 1:
+        fwd_walk_chunks<SEQ, 1>(sm, r, k, v, w, o, Hs, scale, B, H, T, NT, bh, c_begin, c_end, hh, nx, acc);
+        break;
+    case 2:
+        fwd_walk_chunks<SEQ, 2>(sm, r, k, v, w, o, Hs, scale, B, H, T, NT, bh, c_begin, c_end, hh, nx, acc);
+        break;
+    default:
+        fwd_walk_chunks<SEQ, 3>(sm, r, k, v, w, o, Hs, scale, B, H, T, NT, bh, c_begin, c_end, hh, nx, acc);
+        break;
+    }
+
+    // ---- end of the sequence: the final state ----
+    if (seg == P - 1) {
+#pragma unroll
+        for (int tp = 0; tp < 2; ++tp) {
+            const size_t e = (size_t)(16 * W + lr) * KD + 32 * hh + 16 * tp + 4 * lq;
+            *reinterpret_cast<uint2*>(Hs + (size_t)bh * (NT + 1) * KD * KD + (size_t)NT * KD * KD + e) =
+                make_uint2(pk2(acc[tp][0], acc[tp][1]), pk2(acc[tp][2], acc[tp][3]));
+            if (hT)
+                *reinterpret_cast<float4*>(hT + sbase + e) =
+                    make_float4(acc[tp][0], acc[tp][1], acc[tp][2], acc[tp][3]);
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// forward pre-pass: the end states of runs of chunks ("pieces")
+// ---------------------------------------------------------------------------
+// Segment p of the output walk starts from the state entering its first chunk.  Each of the
+// segments 0..P-2 is cut into SUB pieces of at most NCS chunks; one workgroup per (b,h, piece)
+// walks its chunks from a zero state, two chunks (PSPAN = 128 tokens) per step,
+//   S = diag(e^{G_end}) S + sum_tau (k_tau e^{G_end - G_tau}) v_tau^T        [MFMA]
+// with G the cumulative log-decay over the step, and writes the piece's end state S_q (fp32
+// [64][64]) and total log2-decay A_q ([64]).  Only k, v and w are read.  Per step, thread
+// (part, i) scans the log-decay of channel i over the tokens 16 part .. 16 part + 15 and forms
+// those tokens' k e^{G_end - G} itself, written channel-major (two 16-byte stores) as the
+// MFMA's A operand: no cumulative-decay tile.  The raw tiles are double-buffered, so a step
+// takes two barriers (piece_steps: the next step's scan runs beside this step's state
+// update; four before, 78.4 -> 76.8 us at config 5).  The exponents G_end - G_tau are never
+// positive, whatever the step's length, so the end state needs none of the walk's 64-token
+// references; 128-token steps halve the barriers per token (86.7 against 89.2 us at config 5
+// with one 64-token chunk per step; loads two steps ahead measured no faster, and a plain
+// read stream of the same shape, one workgroup per CU, takes 59 us).  With 132 KB of LDS a
+// piece takes a CU to itself; prepass_pieces caps the pieces at one per CU.
 template <bool SEQ>
 __global__ void __launch_bounds__(NTHR_W)
 wkv6_fwd_pieces(const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
@@ -2407,11 +2498,63 @@ __device__ __forceinline__ void bwd_loop_walk(
     }
 }
 
+// The state gradient that the chunks c0 .. NT-1 hand to the left, from dhT (or zero): the thread's
+// four elements dS[ch][tj .. tj + 3].  Waves 0-7 of the loop's sixteen run the piece steps, the
+// others pass the same barriers; LDS is free again after it.
+template <bool SEQ>
+__device__ __forceinline__ f32x4 bwd_suffix(unsigned char* smem, const uint16_t* __restrict__ r,
+                                            const uint16_t* __restrict__ w,
+                                            const uint16_t* __restrict__ dO,
+                                            const float* __restrict__ dhT, float scale, int bh,
+                                            int c0, int B, int H, int T, int NT, int ch, int tj) {
+    PieceSmem& ps = *reinterpret_cast<PieceSmem*>(smem);
+    const int nsteps = (NT - c0 + 1) / 2;
+    float* x = reinterpret_cast<float*>(smem);              // after the steps: dS [64][PST], decay [64]
+    if (threadIdx.x < NTHR_W) {
+        const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, lr = lane & 15, lq = lane >> 4;
+        const int row = threadIdx.x >> 3, c8 = (threadIdx.x & 7) * 8, PW = wv >> 1, hh = wv & 1;
+        const size_t rs = tok_rs<SEQ>(B, H);
+        PieceLoads nx;
+        auto issue = [&](int m) {
+            const int t0 = (c0 + 2 * m) * CL, nv = min(PSPAN, T - t0);
+            const size_t base = tok_base<SEQ>(bh, t0, B, H, T);
+            const size_t dbase = tok_base<false>(bh, t0, B, H, T);
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int rrow = min(row + 64 * h, nv - 1);
+                nx.x[h] = *reinterpret_cast<const uint4*>(r + base + (size_t)rrow * rs + c8);
+                nx.w[h] = *reinterpret_cast<const uint4*>(w + base + (size_t)rrow * rs + c8);
+                nx.y[h] = *reinterpret_cast<const uint4*>(dO + dbase + (size_t)rrow * KD + c8);
+            }
+        };
+        auto nvalid = [&](int m) { return min(PSPAN, T - (c0 + 2 * m) * CL); };
+        f32x4 st[2] = {};
+        float gsum = 0.f;
+        piece_steps<SEQ, true>(ps, nx, nsteps, issue, nvalid, st, gsum);
+#pragma unroll
+        for (int tp = 0; tp < 2; ++tp)
+#pragma unroll
+            for (int rr = 0; rr < 4; ++rr)
+                x[(16 * PW + 4 * lq + rr) * PST + 32 * hh + 16 * tp + lr] = scale * st[tp][rr];
+        if (wv == 7) x[KD * PST + lane] = gsum;
+    } else {
+        for (int i = 0; i < PIECE_BARRIERS(nsteps); ++i) __syncthreads();
+    }
+    __syncthreads();
+    f32x4 d = *reinterpret_cast<const f32x4*>(x + ch * PST + tj);
+    const float e = ex2(x[KD * PST + ch]);
+    if (dhT) d += e * *reinterpret_cast<const f32x4*>(dhT + ch * KD + tj);
+    __syncthreads();
+    return d;
+}
+
 // SEQ as for wkv6_bwd_chunk_grads.  One workgroup per (b,h, segment) (P segments of ceil(NT/P)
 // chunks; P = 1 when B*H fills the device): segment p starts from dhT (p = P-1) or dSend[b,h][p]
 // (wkv6_bwd_fold) and writes dh0 if p = 0.  du_part gets one 64-vector per (b,h, segment)
 // ([h][b][p][i]).  The 16 waves: wave 4W + col owns token block W and channel column col.
-template <bool SEQ>
+// PRE: the segment forms its starting state gradient itself, from dhT and the chunks after it (as
+// wkv6_fwd_walk's PRE).
+template <bool SEQ, bool PRE>
 __global__ void __launch_bounds__(NTHR_L)
 wkv6_bwd_loop(const uint16_t* __restrict__ r, const uint16_t* __restrict__ k,
               const uint16_t* __restrict__ v, const uint16_t* __restrict__ w,
@@ -2432,6 +2575,12 @@ wkv6_bwd_loop(const uint16_t* __restrict__ r, const uint16_t* __restrict__ k,
     LaneOfs o = lane_ofs(threadIdx.x & 63, threadIdx.x >> 6);
     GlobOfs go_ = glob_ofs<SEQ>(threadIdx.x, B, H);
 
+    f32x4 Dst = {};                                         // dS[ch][t4 + rr]
+    if constexpr (PRE) {
+        if (c_hi < NT)
+            Dst = bwd_suffix<SEQ>(smem_raw, r, w, dO, dhT ? dhT + sbase : nullptr, scale, bh, c_hi, B, H, T,
+                                  NT, ch0, t40);
+    }
     LoopPrefetch pf;
     loop_issue<SEQ, 0>(pf, r, k, v, w, dO, Hs, bh, c_hi - 1, B, H, T, NT, threadIdx.x, go_);
     loop_issue<SEQ, 1>(pf, r, k, v, w, dO, Hs, bh, c_hi - 1, B, H, T, NT, threadIdx.x, go_);
@@ -2440,8 +2589,7 @@ wkv6_bwd_loop(const uint16_t* __restrict__ r, const uint16_t* __restrict__ k,
     __syncthreads();
     GradLane gl;
     gl.ulane[0] = scale * load_u(u, u_dtype, h * KD + ch0);
-    f32x4 Dst = {};                                         // dS[ch][t4 + rr]
-    {
+    if (!PRE || c_hi >= NT) {
         // dhT for the last segment, else what the later segments hand this one
         const float* d0 = seg + 1 < P ? dSend + ((size_t)bh * (P - 1) + seg) * KD * KD
                                       : (dhT ? dhT + sbase : nullptr);
@@ -2580,16 +2728,18 @@ inline void mark(void* const* ev, int i, hipStream_t s) {
 // The reverse walk's workspace: du partials per (b,h, segment), then (P > 1) the backward
 // pieces' dS_q and A_q and the segments' starting state gradients dS_end.
 inline size_t bwd_walk_workspace_bytes(int64_t BH, int64_t NT) {
-    const int P = bwd_walk_segments(BH, NT);
+    const WalkPlan plan = bwd_walk_plan(BH, NT);
+    const int P = plan.P;
     size_t n = round_up((size_t)(BH * P) * KD * 4);
-    if (P > 1) {
+    if (P > 1 && !plan.pre) {
         const size_t np = (size_t)(BH * (P - 1) * prepass_pieces(BH, NT, P, PIECE_TARGET).sub);
         n += round_up(np * KD * KD * 4) + round_up(np * KD * 4) + round_up((size_t)(BH * (P - 1)) * KD * KD * 4);
     }
     return n;
 }
 inline size_t fwd_workspace_bytes(int64_t BH, int64_t NT, int64_t max_pieces) {
-    const int P = walk_segments(BH, NT);
+    const WalkPlan plan = fwd_walk_plan(BH, NT);
+    const int P = plan.pre ? 1 : plan.P;             // a walk that forms its own start states needs none
     const size_t n = (size_t)(BH * (P - 1) * prepass_pieces(BH, NT, P, max_pieces).sub);
     const size_t starts = (size_t)(BH * (P - 1)) * KD * KD * 4;
     return std::max<size_t>(256, round_up(n * KD * KD * 4) + round_up(n * KD * 4) + round_up(starts));
@@ -2610,7 +2760,7 @@ size_t rwkv6_wkv_workspace_bytes(int64_t B, int64_t H, int64_t T, int64_t K, int
     if (check_shape(B, H, T, K, V) != RWKV6_OK) return 0;
     const size_t BH = (size_t)(B * H), NT = (size_t)(nchunks(T) > 0 ? nchunks(T) : 1);
     if (!for_bwd) return fwd_workspace_bytes((int64_t)BH, nchunks(T), PIECE_TARGET);
-    if (bwd_walk_segments((int64_t)BH, nchunks(T))) return bwd_walk_workspace_bytes((int64_t)BH, nchunks(T));
+    if (bwd_walk_plan((int64_t)BH, nchunks(T)).P) return bwd_walk_workspace_bytes((int64_t)BH, nchunks(T));
     // dHs, du_part per chunk, dS_loc, dec
     return 2 * round_up(BH * NT * KD * KD * 2) + 2 * round_up(BH * NT * KD * 4);
 }
@@ -2633,10 +2783,14 @@ int lds_attributes(hipStream_t stream) {
             size_t bytes;
         };
         const Lds list[] = {
-            {reinterpret_cast<const void*>(wkv6_fwd_walk<false>), sizeof(WalkSmem)},
-            {reinterpret_cast<const void*>(wkv6_fwd_walk<true>), sizeof(WalkSmem)},
-            {reinterpret_cast<const void*>(wkv6_bwd_loop<false>), sizeof(LoopSmem)},
-            {reinterpret_cast<const void*>(wkv6_bwd_loop<true>), sizeof(LoopSmem)},
+            {reinterpret_cast<const void*>(wkv6_fwd_walk<false, false>), sizeof(WalkSmem)},
+            {reinterpret_cast<const void*>(wkv6_fwd_walk<true, false>), sizeof(WalkSmem)},
+            {reinterpret_cast<const void*>(wkv6_fwd_walk<false, true>), WALK_PRE_LDS},
+            {reinterpret_cast<const void*>(wkv6_fwd_walk<true, true>), WALK_PRE_LDS},
+            {reinterpret_cast<const void*>(wkv6_bwd_loop<false, false>), sizeof(LoopSmem)},
+            {reinterpret_cast<const void*>(wkv6_bwd_loop<true, false>), sizeof(LoopSmem)},
+            {reinterpret_cast<const void*>(wkv6_bwd_loop<false, true>), sizeof(LoopSmem)},
+            {reinterpret_cast<const void*>(wkv6_bwd_loop<true, true>), sizeof(LoopSmem)},
             {reinterpret_cast<const void*>(wkv6_bwd_chunk_grads<false>), sizeof(GradSmem)},
             {reinterpret_cast<const void*>(wkv6_bwd_chunk_grads<true>), sizeof(GradSmem)},
         };
@@ -2674,7 +2828,8 @@ int wkv_fwd_impl(const void* r, const void* k, const void* v, const void* w, con
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     const int64_t NT = nchunks(T);
     const int BH = (int)(B * H);
-    const int P = walk_segments(BH, NT);
+    const WalkPlan plan = fwd_walk_plan(BH, NT);
+    const int P = plan.P;
     const Pieces pc = prepass_pieces(BH, NT, P, max_pieces);
     const int npieces = (P - 1) * pc.sub;                  // per sequence
     uint16_t* Hs = reinterpret_cast<uint16_t*>(saved);
@@ -2685,7 +2840,7 @@ int wkv_fwd_impl(const void* r, const void* k, const void* v, const void* w, con
                                              round_up((size_t)BH * npieces * KD * 4));
     if ((st = lds_attributes(s)) != RWKV6_OK) return st;
     mark(phase_events, 0, s);
-    if (P > 1) {
+    if (P > 1 && !plan.pre) {
         hipLaunchKernelGGL((wkv6_fwd_pieces<SEQ>), dim3((unsigned)(BH * npieces)), dim3(NTHR_W), 0, s,
                            (const uint16_t*)k, (const uint16_t*)v, (const uint16_t*)w, Sseg, Aseg,
                            (int)B, (int)H, (int)T, (int)NT, (int)((NT + P - 1) / P), pc.sub, pc.ncs,
@@ -2697,8 +2852,9 @@ int wkv_fwd_impl(const void* r, const void* k, const void* v, const void* w, con
     mark(phase_events, 2, s);
     mark(phase_events, 3, s);
     mark(phase_events, 4, s);
-    hipLaunchKernelGGL((wkv6_fwd_walk<SEQ>), dim3((unsigned)(BH * P)), dim3(NTHR_W),
-                       sizeof(WalkSmem), s, (const uint16_t*)r, (const uint16_t*)k,
+    auto walk = plan.pre ? wkv6_fwd_walk<SEQ, true> : wkv6_fwd_walk<SEQ, false>;
+    hipLaunchKernelGGL(walk, dim3((unsigned)(BH * P)), dim3(NTHR_W),
+                       plan.pre ? WALK_PRE_LDS : sizeof(WalkSmem), s, (const uint16_t*)r, (const uint16_t*)k,
                        (const uint16_t*)v, (const uint16_t*)w, u, u_dtype, h0, (uint16_t*)o, Hs,
                        hT, Sstart, scale, (int)B, (int)H, (int)T, (int)NT, P);
     mark(phase_events, 5, s);
@@ -2747,13 +2903,14 @@ int wkv_bwd_impl(const void* r, const void* k, const void* v, const void* w, con
         for (int i = 1; i <= 7; ++i) mark(phase_events, i, s);
         return launch_status();
     }
-    if (const int P = bwd_walk_segments(BH, NT)) {
+    const WalkPlan plan = bwd_walk_plan(BH, NT);
+    if (const int P = plan.P) {
         // one reverse walk per (b,h, segment): gradients and state gradients in one pass; with
         // P > 1 segments the pieces of segments 1..P-1 and their fold first give each segment
         // its starting state gradient
         du_part = reinterpret_cast<float*>(workspace);
         const float* dSend = nullptr;
-        if (P > 1) {
+        if (P > 1 && !plan.pre) {
             const Pieces pc = prepass_pieces(BH, NT, P, PIECE_TARGET);
             const int npieces = (P - 1) * pc.sub;
             float* dSp = reinterpret_cast<float*>(reinterpret_cast<char*>(du_part) +
@@ -2777,7 +2934,8 @@ int wkv_bwd_impl(const void* r, const void* k, const void* v, const void* w, con
         }
         mark(phase_events, 3, s);
         mark(phase_events, 4, s);
-        hipLaunchKernelGGL(wkv6_bwd_loop<SEQ>, dim3((unsigned)(BH * P)), dim3(NTHR_L), sizeof(LoopSmem), s,
+        auto loop = plan.pre ? wkv6_bwd_loop<SEQ, true> : wkv6_bwd_loop<SEQ, false>;
+        hipLaunchKernelGGL(loop, dim3((unsigned)(BH * P)), dim3(NTHR_L), sizeof(LoopSmem), s,
                            (const uint16_t*)r, (const uint16_t*)k, (const uint16_t*)v,
                            (const uint16_t*)w, u, u_dtype, (const uint16_t*)dO, dhT, Hs,
                            (uint16_t*)dr, (uint16_t*)dk, (uint16_t*)dv, (uint16_t*)dw, du_part, dh0,
@@ -2825,7 +2983,7 @@ int wkv_bwd_impl(const void* r, const void* k, const void* v, const void* w, con
 // forward's only scratch, the end states of its pre-pass pieces (S_q fp32 [64][64] and A_q
 // fp32 [64] per piece) and the segments' start states (fp32 [64][64] per segment after the
 // first), lives in this file-scope device array instead of the caller's workspace.
-// walk_segments() gives B*H*P <= 256 when P > 1, so B*H*(P-1) < 256, and
+// walk_plan() gives B*H*P <= 256 when P > 1, so B*H*(P-1) < 256, and
 // this entry caps the pieces at WKV_SCRATCH_SEGS (fewer, longer pieces than with a workspace
 // when the cap binds): WKV_SCRATCH_BYTES covers every shape.
 // Each GPU holds its own copy for the life of the process; calls on one GPU share it (the
@@ -2874,6 +3032,12 @@ int rwkv6_wkv_fwd_noalloc(const void* r, const void* k, const void* v, const voi
     if ((st = scratch_address(reinterpret_cast<hipStream_t>(stream), &ws)) != RWKV6_OK) return st;
     return wkv_fwd_impl<false>(r, k, v, w, u, u_dtype, h0, o, hT, saved, ws, B, H, T, K, V, scale,
                                stream, nullptr, WKV_SCRATCH_SEGS);
+}
+
+int rwkv6_wkv_plan(int64_t B, int64_t H, int64_t T, int for_bwd) {
+    if (check_shape(B, H, T, KD, KD) != RWKV6_OK || T == 0) return 0;
+    const WalkPlan p = for_bwd ? bwd_walk_plan(B * H, nchunks(T)) : fwd_walk_plan(B * H, nchunks(T));
+    return p.pre ? -p.P : p.P;
 }
 
 int rwkv6_wkv_fwd_ex(const void* r, const void* k, const void* v, const void* w, const void* u,

@@ -321,3 +321,38 @@ def test_wkv_seqfirst_with_state(pkg):
     ref = dict(o=o_ref, hT=hT_ref, dr=gr["dr"], dk=gr["dk"], dv=gr["dv"], du=gr["du"],
                dw=gr["dw"] * w_hf, dh0=gr["dh0"])
     _compare(got, ref, ["o", "hT", "dr", "dk", "dv", "dw", "du", "dh0"])
+
+
+# The plans of short and few sequences (rwkv6_wkv_plan: forward, backward): segments that form
+# their own start states (negative), with one whole and one ragged last chunk, one-chunk and
+# several-chunk segments, an odd number of chunks before the last segment; the pre-pass over
+# short segments; the chunk-parallel backward; both sides of the line between them.
+@pytest.mark.parametrize("shape,plan", [
+    ((1, 8, 100), (1, -2)), ((1, 8, 65), (1, -2)), ((2, 8, 512), (-8, -8)), ((1, 8, 777), (-13, 0)),
+    ((2, 32, 1001), (-4, -4)), ((4, 32, 500), (-2, -2)), ((3, 32, 700), (-2, -2)),
+    ((1, 32, 2048), (8, 8)), ((1, 16, 64 * 30 + 1), (16, 16))])
+@pytest.mark.parametrize("seq_first", [False, True])
+def test_wkv_plans(pkg, shape, plan, seq_first):
+    B, H, T = shape
+    L = pkg._lib.load()
+    assert (L.rwkv6_wkv_plan(B, H, T, 0), L.rwkv6_wkv_plan(B, H, T, 1)) == plan
+    x = _inputs(B, H, T, seed=B + H + T)
+    if not seq_first:
+        got = run_gpu(pkg, x, 0.5, True, True)
+        again = run_gpu(pkg, x, 0.5, True, True)
+        assert all(np.array_equal(got[n], again[n]) for n in got)
+        ref = run_oracle(x, 0.5, True, True)
+        _compare(got, ref, ["o", "hT", "dr", "dk", "dv", "dw", "du", "dh0"])
+        return
+    dev = torch.device("cuda:0")
+    tb = lambda t: t.permute(2, 0, 1, 3).reshape(T, B, H * 64).contiguous()
+    decay = torch.log(-x["w"].float()).to(torch.bfloat16)
+    x["w"] = -torch.exp(decay.float())
+    leaves = [t.to(dev).requires_grad_(True) for t in (tb(x["r"]), tb(x["k"]), tb(x["v"]), tb(decay), x["u"], x["h0"])]
+    o, hT = pkg.wkv6_seqfirst(*leaves[:5], H, scale=1.0, initial_state=leaves[5], output_final_state=True)
+    g = torch.autograd.grad([o, hT], leaves, [x["do"].to(dev), x["dht"].to(dev)])
+    hf = lambda t: _n(t.view(T, B, H, 64).permute(1, 2, 0, 3))
+    got = dict(o=_n(o), hT=_n(hT), dr=hf(g[0]), dk=hf(g[1]), dv=hf(g[2]), dw=hf(g[3]), du=_n(g[4]), dh0=_n(g[5]))
+    ref = run_oracle(x, 1.0, True, True)
+    ref["dw"] = ref["dw"] * _n(x["w"])
+    _compare(got, ref, ["o", "hT", "dr", "dk", "dv", "dw", "du", "dh0"])
