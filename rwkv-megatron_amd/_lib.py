@@ -117,6 +117,28 @@ def bind(L: ctypes.CDLL, path: str) -> ctypes.CDLL:
     return L
 
 
+_native = None
+
+
+def native():
+    """The autograd functions over the library (csrc/autograd.cpp), loaded once."""
+    global _native
+    if _native is None:
+        load()                              # the missing- or stale-library messages come first
+        try:
+            from . import _native as mod
+        except ImportError as e:
+            raise RuntimeError(f"{HERE}/_native.so cannot be loaded ({e}): build it with "
+                               "`python rwkv-megatron_amd/build.py`") from e
+        if mod.ABI_VERSION != ABI_VERSION:
+            raise RuntimeError(f"{mod.__file__} was built for ABI version {mod.ABI_VERSION}, these "
+                               f"bindings expect {ABI_VERSION}: rebuild it with "
+                               "`python rwkv-megatron_amd/build.py`")
+        mod.set_error(Rwkv6Error)
+        _native = mod
+    return _native
+
+
 def check(status: int, what: str) -> None:
     if status == RWKV6_OK:
         return

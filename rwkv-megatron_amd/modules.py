@@ -48,7 +48,7 @@ import torch
 import torch.nn.functional as F
 from torch import nn
 
-from . import channelmix, timemix
+from . import _lib, channelmix, timemix
 from .wkv import chunk_rwkv6, wkv6_seqfirst
 
 
@@ -88,51 +88,9 @@ def _ramp(C, layer_id, n_layers, device):
     return 1.0 - torch.pow(ddd, ratio)
 
 
-def _splitk_wgrad(dy: torch.Tensor, x: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
-    """dW = dy^T x for dy [N, O], x [N, I] (N = tokens), fp32-accumulated.
-
-    A projection's weight gradient has a small output (O x I, e.g. 2048 x 2048 = 64 tiles
-    of 256 x 256) and a long reduction (16 K tokens): one GEMM occupies a quarter of the
-    256 CUs.  The tokens are split into s chunks (s doubles while the tile count stays below
-    512, at most 4: measured on MI355X at 16 K tokens, a 2048 x 2048 dW takes 155 us with
-    s = 4 against 170 us with s = 8, whose partial sum reads twice the bytes), the chunks run
-    as one batched GEMM with fp32 outputs, and the partials are summed in a fixed order."""
-    N, O = dy.shape
-    I = x.shape[1]
-    tiles = -(-O // 256) * -(-I // 256)
-    s = 1
-    while s < 4 and tiles * s < 512 and N % (2 * s) == 0:
-        s *= 2
-    if s == 1:
-        return (dy.t() @ x).to(dtype)
-    part = torch.bmm(dy.view(s, N // s, O).transpose(1, 2), x.view(s, N // s, I),
-                     out_dtype=torch.float32)
-    return timemix.sum_partials(part, dtype)
-
-
-class _LinearFn(torch.autograd.Function):
-    """y = x W^T; backward dx = dy W on hipBLASLt, dW by the split-token GEMM above."""
-
-    @staticmethod
-    def forward(ctx, x, w):
-        wc = w.to(x.dtype)
-        ctx.save_for_backward(x, wc)
-        ctx.w_dtype = w.dtype
-        return F.linear(x, wc)
-
-    @staticmethod
-    def backward(ctx, dy):
-        x, wc = ctx.saved_tensors
-        dy2 = dy.reshape(-1, dy.shape[-1]).contiguous()
-        dx = (dy2 @ wc).view(x.shape) if ctx.needs_input_grad[0] else None
-        dw = None
-        if ctx.needs_input_grad[1]:
-            dw = _splitk_wgrad(dy2, x.reshape(-1, x.shape[-1]).contiguous(), ctx.w_dtype)
-        return dx, dw
-
-
 class _Linear(nn.Module):
-    """Column/RowParallelLinear at TP=1: weight [out, in], y = x @ W^T, optional bias.
+    """Column/RowParallelLinear at TP=1: weight [out, in], y = x @ W^T, optional bias; the weight
+    gradient split over the tokens (csrc/autograd.cpp).
 
     The weight is initialised by the config's Megatron init callable (``init_attr``:
     ``init_method`` or ``output_layer_init_method``) when it has one, else normal(0, std);
@@ -155,7 +113,7 @@ class _Linear(nn.Module):
                     nn.init.normal_(self.weight, 0.0, std)
 
     def forward(self, x):
-        y = _LinearFn.apply(x, self.weight)
+        y = _lib.native().linear(x, self.weight)
         if self.bias is None:
             return y, None
         b = self.bias.to(y.dtype)
@@ -174,10 +132,11 @@ class LayerNorm(nn.LayerNorm):
 
 class OutputLayer(nn.Linear):
     """The untied output head (rwkv6_model.py, output_layer) as y = x W^T with the parameter cast
-    to the activations' dtype; the weight gradient by the split-token GEMM of _LinearFn."""
+    to the activations' dtype; the weight gradient by the split-token GEMM
+    of csrc/autograd.cpp."""
 
     def forward(self, x):
-        return _LinearFn.apply(x, self.weight)
+        return _lib.native().linear(x, self.weight)
 
 
 class GroupNorm(nn.Module):

@@ -12,6 +12,8 @@
   of :341 disappears; ``group_norm``: the same kernels without the gate (GroupNorm.forward,
   :90-97).
 
+The autograd functions are csrc/autograd.cpp's; the Functions here are the bottlenecks' general
+path, for ranks and sizes the end-to-end kernels (rwkv6_lora_down_fwd / _up_fwd / _bwd) do not take.
 Every function raises if the HIP library is missing; there is no fallback.
 """
 from __future__ import annotations
@@ -48,68 +50,6 @@ def _param(t: torch.Tensor):
 def _ptrs(ts):
     """Host array of device pointers (the C ABI's `void* const*` arguments)."""
     return (ctypes.c_void_p * len(ts))(*[t.data_ptr() for t in ts])
-
-
-# The bottlenecks that the end-to-end kernels (rwkv6_lora_down_fwd / _up_fwd / _bwd) take, as
-# (expansion, rank, with the token-shift lerp); any other runs the general path.  A thread's 64
-# token rows must lie within 32-bit byte offsets there, hence the bound on B*C.
-_FUSED = {(NE, 32, True), (1, 64, False)}
-
-
-def _fused(E, R, lerp, B, C):
-    return (E, R, lerp) in _FUSED and C % 64 == 0 and B * C <= 1 << 23
-
-
-def _weights(w_down, w_up):
-    """Both weights in one dtype code, as the kernels read them: bf16 as they are, a pair of fp32
-    ones too (rounded to bf16 inside the kernels), anything else rounded to bf16 here."""
-    if w_down.dtype == w_up.dtype == torch.float32:
-        return _c(w_down), _c(w_up), _lib.RWKV6_F32
-    return _c(w_down.to(torch.bfloat16)), _c(w_up.to(torch.bfloat16)), _lib.RWKV6_BF16
-
-
-def _lora_fwd(x, maa, w_down, w_up, bias):
-    """neck and the E outputs of a bottleneck of _FUSED; maa None: no token-shift lerp."""
-    T, B, C = x.shape
-    E, R = w_down.shape[1], w_down.shape[2]
-    L, dev, st = _lib.load(), x.device, _stream(x.device)
-    wd, wu, wdt = _weights(w_down, w_up)
-    m, mdt = (None, 0) if maa is None else _param(maa)
-    b, bdt = _param(bias)
-    neck = torch.empty(T * B, E * R, dtype=torch.bfloat16, device=dev)
-    out = tuple(torch.empty(T, B, C, dtype=torch.bfloat16, device=dev) for _ in range(E))
-    _lib.check(L.rwkv6_lora_down_fwd(_p(x), _p(m), mdt, _p(wd), wdt, _p(neck), T, B, C, E, R, st),
-               "rwkv6_lora_down_fwd")
-    _lib.check(L.rwkv6_lora_up_fwd(None if maa is None else _p(x), _p(neck), _p(wu), wdt, _p(b), bdt,
-                                   _ptrs(out), T, B, C, E, R, st), "rwkv6_lora_up_fwd")
-    return neck, out
-
-
-def _grad_like(t):
-    """A parameter gradient's buffer: bf16 for a bf16 parameter, fp32 for any other."""
-    bf = t.dtype == torch.bfloat16
-    return (torch.empty(t.shape, dtype=torch.bfloat16 if bf else torch.float32, device=t.device),
-            _lib.RWKV6_BF16 if bf else _lib.RWKV6_F32)
-
-
-def _lora_bwd(x, maa, w_down, w_up, bias, neck, d_out):
-    """Gradients (dx, d_maa or None, d_w_down, d_w_up, d_bias) of _lora_fwd, parameter gradients
-    in the parameters' dtypes."""
-    T, B, C = x.shape
-    E, R = w_down.shape[1], w_down.shape[2]
-    L, dev = _lib.load(), x.device
-    wd, wu, wdt = _weights(w_down, w_up)
-    m, mdt = (None, 0) if maa is None else _param(maa)
-    b, bdt = _param(bias)
-    dx = torch.empty_like(x)
-    d_maa = None if maa is None else _grad_like(maa)[0]
-    (d_wd, ddt), (d_wu, udt), (d_b, _) = _grad_like(w_down), _grad_like(w_up), _grad_like(bias)
-    ws = torch.empty(L.rwkv6_lora_bwd_workspace_bytes(T, B, C, E, R), dtype=torch.uint8, device=dev)
-    _lib.check(L.rwkv6_lora_bwd(_p(x), _p(m), mdt, _ptrs(d_out), _p(neck), _p(wd), _p(wu), wdt, _p(b), bdt,
-                                _p(dx), _p(d_maa), _p(d_wd), ddt, _p(d_wu), udt, _p(d_b), _p(ws), T, B, C,
-                                E, R, _stream(dev)), "rwkv6_lora_bwd")
-    return (dx, None if maa is None else d_maa.to(maa.dtype), d_wd.to(w_down.dtype), d_wu.to(w_up.dtype),
-            d_b.to(bias.dtype))
 
 
 def _check_act(name, x, ndim):
@@ -160,29 +100,6 @@ def col_sum(x, dtype):
     return out
 
 
-def gn_gate_fwd(o, head_first, g_pre, gamma, beta, eps):
-    """GroupNorm over heads of 64 channels times silu(g_pre); g_pre None: GroupNorm alone."""
-    if head_first:
-        B, H, T, K = o.shape
-    else:
-        T, B, C = o.shape
-        K = 64
-        H = C // K
-    o = _c(o)
-    g_pre = None if g_pre is None else _c(g_pre)
-    ga, pdt = _param(gamma)
-    be, pdt_b = _param(beta)
-    if pdt_b != pdt:
-        be = _c(be.to(ga.dtype))
-    y = torch.empty(T, B, H * K, dtype=torch.bfloat16, device=o.device)
-    mean = torch.empty(T * B * H, dtype=torch.float32, device=o.device)
-    rstd = torch.empty_like(mean)
-    _lib.check(_lib.load().rwkv6_gn_gate_fwd(_p(o), int(head_first), _p(g_pre), _p(ga), _p(be), pdt,
-                                             float(eps), _p(y), _p(mean), _p(rstd), T, B, H, K,
-                                             _stream(o.device)), "rwkv6_gn_gate_fwd")
-    return y, mean, rstd
-
-
 # ---------------------------------------------------------------------------
 # autograd Functions
 # ---------------------------------------------------------------------------
@@ -227,10 +144,6 @@ class _TokenShiftMix(torch.autograd.Function):
         R = w_down.shape[-1]
         N = T * B
         x = _c(x)
-        if _fused(w_down.shape[1], R, True, B, C):
-            neck, mixed = _lora_fwd(x, maa, w_down, w_up, bias)
-            ctx.save_for_backward(x, maa, w_down, w_up, bias, neck)
-            return mixed
         wd = w_down.to(torch.bfloat16).reshape(C, NE * R)
         wut = w_up.to(torch.bfloat16).transpose(1, 2).contiguous()             # [5, C, R]
         xxx = shift_lerp(x, maa)
@@ -245,16 +158,13 @@ class _TokenShiftMix(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, *d_mixed):
-        x, maa, w_down, w_up, bias, *rest = ctx.saved_tensors
+        x, maa, w_down, w_up, bias, xxx, neck, wut = ctx.saved_tensors
         T, B, C = x.shape
         R = w_down.shape[-1]
         N = T * B
         L = _lib.load()
         dev = x.device
         d_mixed = [torch.zeros_like(x) if d is None else _c(d.to(torch.bfloat16)) for d in d_mixed]
-        if len(rest) == 1:
-            return _lora_bwd(x, maa, w_down, w_up, bias, rest[0], d_mixed)
-        xxx, neck, wut = rest
         b, pdt = _param(bias)
         d_mexp = torch.empty(NE, N, C, dtype=torch.bfloat16, device=dev)
         dd = torch.empty(N, C, dtype=torch.bfloat16, device=dev)
@@ -297,10 +207,6 @@ class _Lora(torch.autograd.Function):
         E, R = w_down.shape[1], w_down.shape[2]
         N = T * B
         x = _c(x)
-        if _fused(E, R, False, B, C):
-            neck, (out,) = _lora_fwd(x, None, w_down, w_up, bias)
-            ctx.save_for_backward(x, w_down, w_up, bias, neck)
-            return out.view(T, B, 1, C)
         wd = w_down.to(torch.bfloat16).reshape(C, E * R)
         wut = w_up.to(torch.bfloat16).transpose(1, 2).contiguous()             # [E, C, R]
         neck = _c(torch.tanh(x.view(N, C) @ wd))                                # [N, E*R]
@@ -313,14 +219,10 @@ class _Lora(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, d_out):
-        x, w_down, w_up, bias, neck, *rest = ctx.saved_tensors
+        x, w_down, w_up, bias, neck, wut = ctx.saved_tensors
         T, B, C = x.shape
         E, R = w_down.shape[1], w_down.shape[2]
         N = T * B
-        if not rest:
-            dx, _, d_wd, d_wu, d_b = _lora_bwd(x, None, w_down, w_up, bias, neck, [_c(d_out.to(torch.bfloat16))])
-            return dx, d_wd, d_wu, d_b
-        (wut,) = rest
         g = _c(d_out.to(torch.bfloat16)).view(N, E, C)
         d_bias = col_sum(g.view(N, E * C), bias.dtype).view(E, C)              # [E, C]
         neck3 = neck.view(N, E, R)
@@ -339,7 +241,8 @@ def lora(x, w_down, w_up, bias):
     _check_act("x", x, 3)
     if w_down.dim() != 3 or w_up.dim() != 3 or w_down.shape[1] != w_up.shape[0]:
         raise ValueError("expected w_down [C,E,R], w_up [E,R,C]")
-    return _Lora.apply(x, w_down, w_up, bias)
+    out = _lib.native().decay_lora(x, w_down, w_up, bias)
+    return _Lora.apply(x, w_down, w_up, bias) if out is None else out.unsqueeze(2)
 
 
 def decay_lora(x, w_down, w_up, bias):
@@ -347,54 +250,16 @@ def decay_lora(x, w_down, w_up, bias):
     _check_act("x", x, 3)
     if w_down.dim() != 3 or w_down.shape[1] != 1:
         raise ValueError("decay_lora expects the E = 1 bottleneck (w_down [C,1,R])")
-    return _Lora.apply(x, w_down, w_up, bias).view(x.shape)
+    out = _lib.native().decay_lora(x, w_down, w_up, bias)
+    return _Lora.apply(x, w_down, w_up, bias).view(x.shape) if out is None else out
 
 
 def token_shift_mix(x, maa, w_down, w_up, bias):
     """Returns the five [T,B,C] mixes (w, k, v, r, g), the inputs of RWKV6TimeMix's
     projections (:440-452)."""
     _check_act("x", x, 3)
-    return _TokenShiftMix.apply(x, maa, w_down, w_up, bias)
-
-
-class _GroupNormGate(torch.autograd.Function):
-    """y = GroupNorm_heads(o) * silu(g_pre), or GroupNorm alone when g_pre is None."""
-
-    @staticmethod
-    def forward(ctx, o, head_first, g_pre, gamma, beta, eps):
-        y, mean, rstd = gn_gate_fwd(o, head_first, g_pre, gamma, beta, eps)
-        ctx.save_for_backward(o, g_pre, gamma, beta, mean, rstd)
-        ctx.head_first = head_first
-        return y
-
-    @staticmethod
-    def backward(ctx, dy):
-        o, g_pre, gamma, beta, mean, rstd = ctx.saved_tensors
-        head_first = ctx.head_first
-        if head_first:
-            B, H, T, K = o.shape
-        else:
-            T, B, C = o.shape
-            K = 64
-            H = C // K
-        L = _lib.load()
-        o, dy = _c(o), _c(dy.to(torch.bfloat16))
-        g_pre = None if g_pre is None else _c(g_pre)
-        ga, pdt = _param(gamma)
-        be, pdt_b = _param(beta)
-        if pdt_b != pdt:
-            be = _c(be.to(ga.dtype))
-        d_o = torch.empty_like(o)
-        d_g = None if g_pre is None else torch.empty_like(g_pre)
-        dgamma = torch.empty(H * K, dtype=ga.dtype, device=o.device)
-        dbeta = torch.empty_like(dgamma)
-        ws = torch.empty(L.rwkv6_gn_gate_bwd_workspace_bytes(T, B, H, K), dtype=torch.uint8,
-                         device=o.device)
-        _lib.check(L.rwkv6_gn_gate_bwd(_p(o), int(head_first), _p(g_pre), _p(ga), _p(be), pdt,
-                                       _p(mean), _p(rstd), _p(dy), _p(d_o), _p(d_g), _p(dgamma),
-                                       _p(dbeta), _p(ws), T, B, H, K, _stream(o.device)),
-                   "rwkv6_gn_gate_bwd")
-        return d_o, None, d_g, dgamma.to(gamma.dtype), dbeta.to(beta.dtype), None
+    out = _lib.native().token_shift_mix(x, maa, w_down, w_up, bias)
+    return _TokenShiftMix.apply(x, maa, w_down, w_up, bias) if out is None else out
 
 
 def group_norm_gate(o, g_pre, gamma, beta, eps, head_first=True):
@@ -425,4 +290,4 @@ def _group_norm(o, g_pre, gamma, beta, eps, head_first):
         raise NotImplementedError("GroupNorm gate supports head size 64 only")
     if g_pre is not None and tuple(g_pre.shape) != (T, B, H * K):
         raise ValueError(f"g_pre must be [T,B,C] = {(T, B, H * K)}, got {tuple(g_pre.shape)}")
-    return _GroupNormGate.apply(o, bool(head_first), g_pre, gamma, beta, float(eps))
+    return _lib.native().group_norm_gate(o, g_pre, gamma, beta, float(eps), bool(head_first))

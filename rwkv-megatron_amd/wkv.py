@@ -16,94 +16,16 @@ same contract (4th argument named ``g``).  Both names are provided here:
   carried state.  bf16 r, k, v, g are used as they are; fp32 / fp16 ones are rounded to
   bf16 on entry (one rounding each, 2^-9 relative), so an fp32 caller gets bf16-operand
   arithmetic, not fp32 arithmetic.  u is used in its own dtype (fp32 or bf16).
-* Backward returns gradients for r, k, v, g, u and initial_state, and accepts a
+* The autograd function is csrc/autograd.cpp's.  Backward returns gradients for r, k, v, g, u and initial_state, and accepts a
   gradient on final_state.
 """
 from __future__ import annotations
-
-import ctypes
 
 import torch
 
 from . import _lib
 
 _HEAD = 64
-
-
-def _stream_ptr(device) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
-
-
-def _p(t):
-    return ctypes.c_void_p(0 if t is None else t.data_ptr())
-
-
-def _aligned(t: torch.Tensor) -> torch.Tensor:
-    t = t.contiguous()
-    if t.data_ptr() % 16:
-        t = t.clone()
-    return t
-
-
-def _bf16(t: torch.Tensor) -> torch.Tensor:
-    return _aligned(t if t.dtype == torch.bfloat16 else t.to(torch.bfloat16))
-
-
-def _u_arg(u: torch.Tensor):
-    if u.dtype == torch.bfloat16:
-        return _aligned(u), _lib.RWKV6_BF16
-    return _aligned(u.float()), _lib.RWKV6_F32
-
-
-class _WKV6(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, r, k, v, w, u, scale, h0, output_final_state):
-        B, H, T, K = r.shape
-        V = v.shape[-1]
-        dev = r.device
-        out_dtype = r.dtype
-        rb, kb, vb, wb = _bf16(r), _bf16(k), _bf16(v), _bf16(w)
-        ua, u_code = _u_arg(u)
-        h0f = None if h0 is None else _aligned(h0.float())
-        L = _lib.load()
-        saved = torch.empty(L.rwkv6_wkv_saved_bytes(B, H, T, K, V), dtype=torch.uint8, device=dev)
-        work = torch.empty(L.rwkv6_wkv_workspace_bytes(B, H, T, K, V, 0), dtype=torch.uint8, device=dev)
-        o = torch.empty(B, H, T, V, dtype=torch.bfloat16, device=dev)
-        hT = torch.empty(B, H, K, V, dtype=torch.float32, device=dev) if output_final_state else None
-        _lib.check(L.rwkv6_wkv_fwd(_p(rb), _p(kb), _p(vb), _p(wb), _p(ua), u_code, _p(h0f), _p(o),
-                                   _p(hT), _p(saved), _p(work), B, H, T, K, V, float(scale),
-                                   _stream_ptr(dev)), "rwkv6_wkv_fwd")
-        ctx.save_for_backward(rb, kb, vb, wb, ua, saved)
-        ctx.meta = (scale, u_code, h0 is not None, u.dtype, out_dtype, r.dtype, k.dtype, v.dtype,
-                    w.dtype, None if h0 is None else h0.dtype)
-        if out_dtype != torch.bfloat16:
-            o = o.to(out_dtype)
-        return o, hT
-
-    @staticmethod
-    def backward(ctx, do, dht):
-        rb, kb, vb, wb, ua, saved = ctx.saved_tensors
-        scale, u_code, has_h0, u_dtype, _, r_dt, k_dt, v_dt, w_dt, h0_dt = ctx.meta
-        B, H, T, K = rb.shape
-        V = vb.shape[-1]
-        dev = rb.device
-        L = _lib.load()
-        dob = _bf16(do) if do is not None else torch.zeros(B, H, T, V, dtype=torch.bfloat16, device=dev)
-        dhtf = None if dht is None else _aligned(dht.float())
-        dr = torch.empty_like(rb)
-        dk = torch.empty_like(kb)
-        dv = torch.empty_like(vb)
-        dw = torch.empty_like(wb)
-        du = torch.empty(H, K, dtype=ua.dtype, device=dev)
-        need_h0 = has_h0 and ctx.needs_input_grad[6]
-        dh0 = torch.empty(B, H, K, V, dtype=torch.float32, device=dev) if need_h0 else None
-        work = torch.empty(L.rwkv6_wkv_workspace_bytes(B, H, T, K, V, 1), dtype=torch.uint8, device=dev)
-        _lib.check(L.rwkv6_wkv_bwd(_p(rb), _p(kb), _p(vb), _p(wb), _p(ua), u_code, _p(dob), _p(dhtf),
-                                   _p(saved), _p(dr), _p(dk), _p(dv), _p(dw), _p(du), _p(dh0), _p(work),
-                                   B, H, T, K, V, float(scale), _stream_ptr(dev)), "rwkv6_wkv_bwd")
-        cast = lambda t, dt: t if t.dtype == dt else t.to(dt)
-        return (cast(dr, r_dt), cast(dk, k_dt), cast(dv, v_dt), cast(dw, w_dt), cast(du, u_dtype),
-                None, None if dh0 is None else cast(dh0, h0_dt), None)
 
 
 def _validate(r, k, v, w, u, initial_state):
@@ -142,10 +64,16 @@ def chunk_rwkv6(r, k, v, g, u, scale=None, initial_state=None, output_final_stat
         raise NotImplementedError("variable-length batches (cu_seqlens) are not supported")
     if not head_first:
         raise NotImplementedError("only the head-first [B,H,T,K] layout is supported")
-    _validate(r, k, v, g, u, initial_state)
     if scale is None or scale == -1:
-        scale = r.shape[-1] ** -0.5
-    return _WKV6.apply(r, k, v, g, u, float(scale), initial_state, bool(output_final_state))
+        scale = _HEAD ** -0.5
+    try:
+        out = _lib.native().wkv6(r, k, v, g, u, initial_state, float(scale), bool(output_final_state))
+    except TypeError:
+        out = None
+    if out is None:                         # an argument does not fit: say which
+        _validate(r, k, v, g, u, initial_state)
+        raise ValueError("WKV6 arguments do not fit together")
+    return out
 
 
 def fused_recurrent_rwkv6(r, k, v, w, u, scale=-1, initial_state=None, output_final_state=False,
@@ -157,56 +85,6 @@ def fused_recurrent_rwkv6(r, k, v, w, u, scale=-1, initial_state=None, output_fi
     return chunk_rwkv6(r, k, v, w, u, scale=scale, initial_state=initial_state,
                        output_final_state=output_final_state, cu_seqlens=cu_seqlens,
                        head_first=head_first)
-
-
-class _WKV6SeqFirst(torch.autograd.Function):
-    """WKV6 on the time-mix module's own layout: r, k, v, decay [T,B,H*64] bf16 (the linear
-    outputs, rwkv6_layer_specs.py:454-457), w = -exp(decay) (:336) applied in the kernels,
-    output o head-first [B,H,T,64] (what GroupNorm*gate reads)."""
-
-    @staticmethod
-    def forward(ctx, r, k, v, decay, u, scale, H, h0, output_final_state):
-        T, B, C = r.shape
-        K = C // H
-        dev = r.device
-        rb, kb, vb, db = _bf16(r), _bf16(k), _bf16(v), _bf16(decay)
-        ua, u_code = _u_arg(u)
-        h0f = None if h0 is None else _aligned(h0.float())
-        L = _lib.load()
-        saved = torch.empty(L.rwkv6_wkv_saved_bytes(B, H, T, K, K), dtype=torch.uint8, device=dev)
-        work = torch.empty(L.rwkv6_wkv_workspace_bytes(B, H, T, K, K, 0), dtype=torch.uint8, device=dev)
-        o = torch.empty(B, H, T, K, dtype=torch.bfloat16, device=dev)
-        hT = torch.empty(B, H, K, K, dtype=torch.float32, device=dev) if output_final_state else None
-        _lib.check(L.rwkv6_wkv_fwd_seqfirst(_p(rb), _p(kb), _p(vb), _p(db), _p(ua), u_code, _p(h0f), _p(o),
-                                            _p(hT), _p(saved), _p(work), B, H, T, K, K, float(scale),
-                                            _stream_ptr(dev)), "rwkv6_wkv_fwd_seqfirst")
-        ctx.save_for_backward(rb, kb, vb, db, ua, saved)
-        ctx.meta = (scale, u_code, H, h0 is not None, u.dtype, r.dtype, k.dtype, v.dtype, decay.dtype,
-                    None if h0 is None else h0.dtype)
-        return o, hT
-
-    @staticmethod
-    def backward(ctx, do, dht):
-        rb, kb, vb, db, ua, saved = ctx.saved_tensors
-        scale, u_code, H, has_h0, u_dt, r_dt, k_dt, v_dt, d_dt, h0_dt = ctx.meta
-        T, B, C = rb.shape
-        K = C // H
-        dev = rb.device
-        L = _lib.load()
-        dob = _bf16(do) if do is not None else torch.zeros(B, H, T, K, dtype=torch.bfloat16, device=dev)
-        dhtf = None if dht is None else _aligned(dht.float())
-        dr, dk, dv, ddec = (torch.empty_like(rb) for _ in range(4))
-        du = torch.empty(H, K, dtype=ua.dtype, device=dev)
-        need_h0 = has_h0 and ctx.needs_input_grad[7]
-        dh0 = torch.empty(B, H, K, K, dtype=torch.float32, device=dev) if need_h0 else None
-        work = torch.empty(L.rwkv6_wkv_workspace_bytes(B, H, T, K, K, 1), dtype=torch.uint8, device=dev)
-        _lib.check(L.rwkv6_wkv_bwd_seqfirst(_p(rb), _p(kb), _p(vb), _p(db), _p(ua), u_code, _p(dob),
-                                            _p(dhtf), _p(saved), _p(dr), _p(dk), _p(dv), _p(ddec), _p(du),
-                                            _p(dh0), _p(work), B, H, T, K, K, float(scale),
-                                            _stream_ptr(dev)), "rwkv6_wkv_bwd_seqfirst")
-        cast = lambda t, dt: t if t.dtype == dt else t.to(dt)
-        return (cast(dr, r_dt), cast(dk, k_dt), cast(dv, v_dt), cast(ddec, d_dt), cast(du, u_dt),
-                None, None, None if dh0 is None else cast(dh0, h0_dt), None)
 
 
 def wkv6_seqfirst(r, k, v, decay, u, num_heads, scale=1.0, initial_state=None,
@@ -226,5 +104,5 @@ def wkv6_seqfirst(r, k, v, decay, u, num_heads, scale=1.0, initial_state=None,
         raise ValueError(f"u must be [H,64], got {tuple(u.shape)}")
     if initial_state is not None and tuple(initial_state.shape) != (B, num_heads, _HEAD, _HEAD):
         raise ValueError("initial_state must be [B,H,64,64]")
-    return _WKV6SeqFirst.apply(r, k, v, decay, u, float(scale), int(num_heads), initial_state,
-                               bool(output_final_state))
+    return _lib.native().wkv6_seqfirst(r, k, v, decay, u, initial_state, float(scale), int(num_heads),
+                                       bool(output_final_state))

@@ -1,0 +1,103 @@
+"""The C++ autograd functions (csrc/autograd.cpp) where a Python autograd function has rules that
+they must keep: saved-tensor hooks, in-place changes of saved tensors, outputs no loss uses,
+inputs that need a copy, function transforms and forward-mode differentiation (refused)."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _ops(pkg):
+    """name -> (function of its leaves, leaves)."""
+    g = torch.Generator().manual_seed(5)
+    bf = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16).to(DEV)
+    T, B, C = 70, 2, 128
+    w = -torch.rand(1, 2, T, 64, generator=g).to(torch.bfloat16).to(DEV)
+    hd = lambda: bf(1, 2, T, 64)
+    tm, cm = pkg.timemix, pkg.channelmix
+    return {
+        "wkv": (lambda r, k, v, w, u, h: pkg.chunk_rwkv6(r, k, v, w, u, 1.0, h, True),
+                [hd(), hd(), hd(), w, bf(2, 64).float(), bf(1, 2, 64, 64).float()]),
+        "seqfirst": (lambda r, k, v, d, u: pkg.wkv6_seqfirst(r, k, v, d, u, 2, output_final_state=True),
+                     [bf(T, B, C), bf(T, B, C), bf(T, B, C), bf(T, B, C), bf(2, 64)]),
+        "mix": (tm.token_shift_mix, [bf(T, B, C), bf(C), bf(C, 5, 32) * 0.05, bf(5, 32, C) * 0.1, bf(5, C)]),
+        "decay": (tm.decay_lora, [bf(T, B, C), bf(C, 1, 64) * 0.05, bf(1, 64, C) * 0.1, bf(1, C)]),
+        "gn": (lambda o, x, ga, be: tm.group_norm_gate(o, x, ga, be, 1e-5), [bf(B, 2, T, 64), bf(T, B, C), bf(C), bf(C)]),
+        "lerp": (cm.cmix_lerp, [bf(T, B, C), bf(2, C)]),
+        "relu": (cm.relu_sq, [bf(T, B, C)]),
+        "gate": (cm.sigmoid_gate, [bf(T, B, C), bf(T, B, C)]),
+        "linear": (pkg._lib.native().linear, [bf(T, B, C), bf(64, C).float()]),
+    }
+
+
+NAMES = ["wkv", "seqfirst", "mix", "decay", "gn", "lerp", "relu", "gate", "linear"]
+
+
+def _outs(o):
+    return [t for t in (o if isinstance(o, (tuple, list)) else (o,)) if t is not None]
+
+
+@pytest.mark.parametrize("name", NAMES)
+def test_saved_tensor_hooks_and_versions(pkg, name):
+    fn, leaves = _ops(pkg)[name]
+    leaves = [t.requires_grad_(True) for t in leaves]
+    base = torch.autograd.grad(sum(t.float().square().sum() for t in _outs(fn(*leaves))), leaves)
+    packed = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: (packed.append(t), t.cpu())[1], lambda t: t.to(DEV)):
+        out = _outs(fn(*leaves))
+    assert packed
+    again = torch.autograd.grad(sum(t.float().square().sum() for t in out), leaves)
+    assert all(torch.equal(a, b) for a, b in zip(base, again))
+    out = _outs(fn(*leaves))
+    with torch.no_grad():
+        leaves[0].add_(1)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        torch.autograd.grad(sum(t.float().square().sum() for t in out), leaves)
+
+
+@pytest.mark.parametrize("name", ["wkv", "seqfirst", "mix", "lerp"])
+def test_unused_outputs_have_zero_gradients(pkg, name):
+    """A loss on one output alone: the same gradients as with zero gradients for the others."""
+    fn, leaves = _ops(pkg)[name]
+    leaves = [t.requires_grad_(True) for t in leaves]
+    n = len(_outs(fn(*leaves)))
+    for i in range(n):
+        out = _outs(fn(*leaves))
+        dy = [torch.ones_like(t) if j == i else torch.zeros_like(t) for j, t in enumerate(out)]
+        want = torch.autograd.grad(out, leaves, dy)
+        got = torch.autograd.grad(_outs(fn(*leaves))[i], leaves, torch.ones_like(out[i]))
+        assert all(torch.equal(a, b) for a, b in zip(want, got))
+
+
+@pytest.mark.parametrize("name", NAMES)
+def test_copied_inputs(pkg, name):
+    """Strided inputs and inputs off the 16-byte grid give the results of their dense copies."""
+    fn, leaves = _ops(pkg)[name]
+
+    def strided(t):
+        return torch.stack([t, t], -1)[..., 0]
+
+    def shifted(t):
+        return torch.cat([t.reshape(-1)[:1], t.reshape(-1)])[1:].view(t.shape)
+
+    def run(ls):
+        ls = [t.detach().requires_grad_(True) for t in ls]
+        out = _outs(fn(*ls))
+        return out + list(torch.autograd.grad(out, ls, [strided(torch.ones_like(t)) for t in out]))
+
+    want = run(leaves)
+    for make in (strided, shifted):
+        assert all(torch.equal(a, b) for a, b in zip(want, run([make(t) for t in leaves])))
+
+
+@pytest.mark.parametrize("name", NAMES)
+def test_transforms_are_refused(pkg, name):
+    fn, leaves = _ops(pkg)[name]
+    with pytest.raises(RuntimeError):
+        torch.func.vmap(fn)(*[torch.stack([t, t]) for t in leaves])
+    with pytest.raises(RuntimeError):
+        torch.func.grad(lambda t: _outs(fn(t, *leaves[1:]))[0].float().sum())(leaves[0])
+    import torch.autograd.forward_ad as fwd
+    with fwd.dual_level(), pytest.raises((RuntimeError, NotImplementedError)):
+        _outs(fn(fwd.make_dual(leaves[0].clone().requires_grad_(True), torch.ones_like(leaves[0])), *leaves[1:]))

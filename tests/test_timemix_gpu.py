@@ -347,11 +347,14 @@ def _bottleneck_case(form, T, B, C, wdt, udt, pdt):
     return [t.to(DEV) for t in (x, maa, wd, wu, bias)], dy
 
 
-def _bottleneck_run(pkg, form, leaves, dy):
+def _bottleneck_run(pkg, form, leaves, dy, general=False):
     leaves = [t.detach().requires_grad_(True) for t in leaves]
     x, maa, wd, wu, bias = leaves
-    out = (pkg.timemix.token_shift_mix(*leaves) if form == "mix"
-           else (pkg.timemix.decay_lora(x, wd, wu, bias),))
+    tm = pkg.timemix
+    if form == "mix":
+        out = tm._TokenShiftMix.apply(*leaves) if general else tm.token_shift_mix(*leaves)
+    else:
+        out = (tm._Lora.apply(x, wd, wu, bias).view(x.shape) if general else tm.decay_lora(x, wd, wu, bias),)
     wrt = leaves if form == "mix" else [x, wd, wu, bias]
     return [t.detach() for t in out] + list(torch.autograd.grad(out, wrt, dy))
 
@@ -374,12 +377,11 @@ def _bottleneck_run(pkg, form, leaves, dy):
     (127, 3, 64, torch.float32, torch.float32, torch.float32),
     (128, 1, 64, torch.float16, torch.bfloat16, torch.float16),
     (1009, 2, 512, torch.bfloat16, torch.bfloat16, torch.bfloat16)])
-def test_bottleneck_kernels_match_the_general_path(pkg, monkeypatch, form, T, B, C, wdt, udt, pdt):
+def test_bottleneck_kernels_match_the_general_path(pkg, form, T, B, C, wdt, udt, pdt):
     leaves, dy = _bottleneck_case(form, T, B, C, wdt, udt, pdt)
     got = _bottleneck_run(pkg, form, leaves, dy)
     again = _bottleneck_run(pkg, form, leaves, dy)
-    monkeypatch.setattr(pkg.timemix, "_FUSED", set())
-    ref = _bottleneck_run(pkg, form, leaves, dy)
+    ref = _bottleneck_run(pkg, form, leaves, dy, general=True)
     torch.cuda.synchronize()
     for i, (a, b, c) in enumerate(zip(got, again, ref)):
         assert a.dtype == c.dtype and a.shape == c.shape and torch.equal(a, b)
