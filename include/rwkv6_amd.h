@@ -80,6 +80,13 @@ int rwkv6_wkv_fwd(const void* r, const void* k, const void* v, const void* w, co
                   void* workspace, int64_t B, int64_t H, int64_t T, int64_t K, int64_t V,
                   float scale, void* stream);
 
+/* The forward without a backward to follow: no chunk states are kept, and a few tokens (decoding)
+ * run as the recurrence itself in fp32.  seq_first: the layouts of rwkv6_wkv_fwd_seqfirst (w is
+ * then the pre-activation decay).  workspace: as rwkv6_wkv_fwd's. */
+int rwkv6_wkv_infer(const void* r, const void* k, const void* v, const void* w, const void* u,
+                    int u_dtype, const float* h0, void* o, float* hT, void* workspace, int seq_first,
+                    int64_t B, int64_t H, int64_t T, int64_t K, int64_t V, float scale, void* stream);
+
 /* Gradients of rwkv6_wkv_fwd for loss terms on o (dO, bf16 [B,H,T,V]) and on the
  * final state (dhT, f32 [B,H,K,V], nullable = zero).  dr, dk, dw: [B,H,T,K] bf16;
  * dv: [B,H,T,V] bf16; du: [H,K] in u_dtype; dh0: [B,H,K,V] f32, nullable. */

@@ -91,25 +91,31 @@ std::vector<int64_t> meta(AutogradContext* ctx) { return ctx->saved_data["m"].to
 struct Wkv6 : torch::autograd::Function<Wkv6> {
     static variable_list forward(AutogradContext* ctx, const Tensor& r, const Tensor& k, const Tensor& v,
                                  const Tensor& w, const Tensor& u, const OptTensor& h0, double scale,
-                                 int64_t heads, bool final_state) {
+                                 int64_t heads, bool final_state, bool grad) {
         const bool seq = heads > 0;
         const int64_t B = r.size(seq ? 1 : 0), H = seq ? heads : r.size(1), T = r.size(seq ? 0 : 2), K = 64;
         const Tensor rb = to_bf16(r), kb = to_bf16(k), vb = to_bf16(v), wb = to_bf16(w);
         const Param ua = param(u);
         const bool state = h0.has_value() && h0->defined();
         const Tensor h0f = state ? to_f32(*h0) : Tensor();
-        const Tensor saved = bytes(rwkv6_wkv_saved_bytes(B, H, T, K, K), rb);
+        const Tensor saved = grad ? bytes(rwkv6_wkv_saved_bytes(B, H, T, K, K), rb) : Tensor();
         const Tensor work = bytes(rwkv6_wkv_workspace_bytes(B, H, T, K, K, 0), rb);
         Tensor o = empty({B, H, T, K}, at::kBFloat16, rb);
         const Tensor hT = final_state ? empty({B, H, K, K}, at::kFloat, rb) : Tensor();
-        auto fn = seq ? rwkv6_wkv_fwd_seqfirst : rwkv6_wkv_fwd;
-        check(fn(ptr(rb), ptr(kb), ptr(vb), ptr(wb), ptr(ua.t), ua.dt, fptr(h0f), ptr(o), fptr(hT), ptr(saved),
-                 ptr(work), B, H, T, K, K, (float)scale, stream_of(rb)),
-              seq ? "rwkv6_wkv_fwd_seqfirst" : "rwkv6_wkv_fwd");
-        ctx->set_materialize_grads(false);
-        ctx->save_for_backward({rb, kb, vb, wb, ua.t, saved});
-        put(ctx, {B, H, T, heads, bits(scale), ua.dt, state, code(r), code(k), code(v), code(w), code(u),
-                  state ? code(*h0) : 0});
+        if (grad) {
+            auto fn = seq ? rwkv6_wkv_fwd_seqfirst : rwkv6_wkv_fwd;
+            check(fn(ptr(rb), ptr(kb), ptr(vb), ptr(wb), ptr(ua.t), ua.dt, fptr(h0f), ptr(o), fptr(hT), ptr(saved),
+                     ptr(work), B, H, T, K, K, (float)scale, stream_of(rb)),
+                  seq ? "rwkv6_wkv_fwd_seqfirst" : "rwkv6_wkv_fwd");
+            ctx->set_materialize_grads(false);
+            ctx->save_for_backward({rb, kb, vb, wb, ua.t, saved});
+            put(ctx, {B, H, T, heads, bits(scale), ua.dt, state, code(r), code(k), code(v), code(w), code(u),
+                      state ? code(*h0) : 0});
+        } else {
+            check(rwkv6_wkv_infer(ptr(rb), ptr(kb), ptr(vb), ptr(wb), ptr(ua.t), ua.dt, fptr(h0f), ptr(o), fptr(hT),
+                                  ptr(work), seq, B, H, T, K, K, (float)scale, stream_of(rb)),
+                  "rwkv6_wkv_infer");
+        }
         if (!seq) o = cast(o, r.scalar_type());
         if (final_state) return {o, hT};
         return {o};
@@ -133,7 +139,7 @@ struct Wkv6 : torch::autograd::Function<Wkv6> {
                  stream_of(rb)),
               seq ? "rwkv6_wkv_bwd_seqfirst" : "rwkv6_wkv_bwd");
         return {cast(dr, type(m[7])), cast(dk, type(m[8])), cast(dv, type(m[9])), cast(dw, type(m[10])),
-                cast(du, type(m[11])), dh0.defined() ? cast(dh0, type(m[12])) : dh0, Tensor(), Tensor(), Tensor()};
+                cast(du, type(m[11])), dh0.defined() ? cast(dh0, type(m[12])) : dh0, Tensor(), Tensor(), Tensor(), Tensor()};
     }
 };
 
@@ -148,6 +154,14 @@ void no_transforms() {
                 "the RWKV-6 kernels' autograd functions do not support torch.func transforms");
 }
 
+// whether a backward can follow (the condition under which torch records the function)
+bool recorded(std::initializer_list<const Tensor*> ts, const OptTensor& h0) {
+    if (!at::GradMode::is_enabled()) return false;
+    for (const Tensor* t : ts)
+        if (t->requires_grad()) return true;
+    return h0 && h0->requires_grad();
+}
+
 // None when an argument does not fit: the caller's own checks then say which and raise.
 py::object wkv6(const Tensor& r, const Tensor& k, const Tensor& v, const Tensor& w, const Tensor& u,
                 const OptTensor& h0, double scale, bool final_state) {
@@ -159,7 +173,8 @@ py::object wkv6(const Tensor& r, const Tensor& k, const Tensor& v, const Tensor&
     if (h0 && (h0->device() != r.device() || h0->sizes() != at::IntArrayRef({r.size(0), r.size(1), 64, 64})))
         return py::none();
     no_transforms();
-    const variable_list out = Wkv6::apply(r, k, v, w, u, h0, scale, (int64_t)0, final_state);
+    const variable_list out = Wkv6::apply(r, k, v, w, u, h0, scale, (int64_t)0, final_state,
+                                            recorded({&r, &k, &v, &w, &u}, h0));
     if (final_state) return py::make_tuple(out[0], out[1]);
     return py::make_tuple(out[0], py::none());
 }
@@ -167,7 +182,8 @@ py::object wkv6(const Tensor& r, const Tensor& k, const Tensor& v, const Tensor&
 py::tuple wkv6_seqfirst(const Tensor& r, const Tensor& k, const Tensor& v, const Tensor& decay, const Tensor& u,
                         const OptTensor& h0, double scale, int64_t heads, bool final_state) {
     no_transforms();
-    const variable_list out = Wkv6::apply(r, k, v, decay, u, h0, scale, heads, final_state);
+    const variable_list out = Wkv6::apply(r, k, v, decay, u, h0, scale, heads, final_state,
+                                            recorded({&r, &k, &v, &decay, &u}, h0));
     if (final_state) return py::make_tuple(out[0], out[1]);
     return py::make_tuple(out[0], py::none());
 }

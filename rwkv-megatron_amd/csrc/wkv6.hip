@@ -475,6 +475,7 @@ __device__ __forceinline__ void walk_issue(WalkPrefetch& f, const uint16_t* __re
 
 // Global stores of chunk c (o from Ot, S_in from Sin[c & 1]).  Issued one
 // chunk late, before the next prefetch: the wait for a prefetch then never waits on a store.
+template <bool SAVE>
 __device__ __forceinline__ void walk_store(const WalkSmem& sm, uint16_t* __restrict__ o,
                                            uint16_t* __restrict__ Hs, int bh, int c, int T,
                                            int NT) {
@@ -487,7 +488,7 @@ __device__ __forceinline__ void walk_store(const WalkSmem& sm, uint16_t* __restr
     // walk and 8 us off the next call's pre-pass at config 5
     __builtin_nontemporal_store(__builtin_bit_cast(u32x4_t, *reinterpret_cast<const uint4*>(&sm.Ot[ro][c8])),
                                 reinterpret_cast<u32x4_t*>(o + ((size_t)bh * T + t0 + ro) * KD + c8));
-    __builtin_nontemporal_store(
+    if constexpr (SAVE) __builtin_nontemporal_store(
         __builtin_bit_cast(u32x4_t, *reinterpret_cast<const uint4*>(&sm.Sin[c & 1][row][c8])),
         reinterpret_cast<u32x4_t*>(Hs + ((size_t)bh * (NT + 1) + c) * KD * KD + row * KD + c8));
 }
@@ -496,7 +497,7 @@ __device__ __forceinline__ void walk_store(const WalkSmem& sm, uint16_t* __restr
 // the operand tiles and, in the products, on token block W = (0, 0, 1, 1, 3, 3, 2, 2)[wv]:
 // both are compile-time here (PB = wv >> 1), so the cross-block loops, the table choices and
 // their offsets are resolved statically; all four instantiations pass the same barriers.
-template <bool SEQ, int PB>
+template <bool SEQ, int PB, bool SAVE>
 __device__ __forceinline__ void fwd_walk_chunks(
         WalkSmem& sm, const uint16_t* __restrict__ r, const uint16_t* __restrict__ k,
         const uint16_t* __restrict__ v, const uint16_t* __restrict__ w,
@@ -716,7 +717,7 @@ __device__ __forceinline__ void fwd_walk_chunks(
         // o and S_in of this chunk, stored after the next chunk's loads were issued: the wait
         // for those at the top of the next iteration leaves these stores in flight (vmcnt
         // counts loads and stores in issue order)
-        walk_store(sm, o, Hs, bh, c, T, NT);
+        walk_store<SAVE>(sm, o, Hs, bh, c, T, NT);
     }
 
 }
@@ -919,7 +920,9 @@ __device__ __forceinline__ void fwd_prefix(unsigned char* smem, const uint16_t* 
 // PRE: segment p >= 1 forms its start state itself, from h0 and the chunks before it (piece
 // steps of 128 tokens), instead of reading it from a pre-pass: one launch instead of three for
 // sequences short enough that re-reading the prefix costs less (walk_plan).
-template <bool SEQ, bool PRE>
+// SAVE: the chunk states go to Hs for a backward (without one they are not stored: 128 of 768 bytes
+// a token and head).
+template <bool SEQ, bool PRE, bool SAVE>
 __global__ void __launch_bounds__(NTHR_W) __attribute__((amdgpu_waves_per_eu(WALK_WPE)))
 wkv6_fwd_walk(const uint16_t* __restrict__ r, const uint16_t* __restrict__ k,
               const uint16_t* __restrict__ v, const uint16_t* __restrict__ w,
@@ -974,16 +977,16 @@ wkv6_fwd_walk(const uint16_t* __restrict__ r, const uint16_t* __restrict__ k,
 
     switch (__builtin_amdgcn_readfirstlane(wv >> 1)) {
     case 0:
-        fwd_walk_chunks<SEQ, 0>(sm, r, k, v, w, o, Hs, scale, B, H, T, NT, bh, c_begin, c_end, hh, nx, acc);
+        fwd_walk_chunks<SEQ, 0, SAVE>(sm, r, k, v, w, o, Hs, scale, B, H, T, NT, bh, c_begin, c_end, hh, nx, acc);
         break;
     case 1:
-        fwd_walk_chunks<SEQ, 1>(sm, r, k, v, w, o, Hs, scale, B, H, T, NT, bh, c_begin, c_end, hh, nx, acc);
+        fwd_walk_chunks<SEQ, 1, SAVE>(sm, r, k, v, w, o, Hs, scale, B, H, T, NT, bh, c_begin, c_end, hh, nx, acc);
         break;
     case 2:
-        fwd_walk_chunks<SEQ, 2>(sm, r, k, v, w, o, Hs, scale, B, H, T, NT, bh, c_begin, c_end, hh, nx, acc);
+        fwd_walk_chunks<SEQ, 2, SAVE>(sm, r, k, v, w, o, Hs, scale, B, H, T, NT, bh, c_begin, c_end, hh, nx, acc);
         break;
     default:
-        fwd_walk_chunks<SEQ, 3>(sm, r, k, v, w, o, Hs, scale, B, H, T, NT, bh, c_begin, c_end, hh, nx, acc);
+        fwd_walk_chunks<SEQ, 3, SAVE>(sm, r, k, v, w, o, Hs, scale, B, H, T, NT, bh, c_begin, c_end, hh, nx, acc);
         break;
     }
 
@@ -992,12 +995,89 @@ wkv6_fwd_walk(const uint16_t* __restrict__ r, const uint16_t* __restrict__ k,
 #pragma unroll
         for (int tp = 0; tp < 2; ++tp) {
             const size_t e = (size_t)(16 * W + lr) * KD + 32 * hh + 16 * tp + 4 * lq;
-            *reinterpret_cast<uint2*>(Hs + (size_t)bh * (NT + 1) * KD * KD + (size_t)NT * KD * KD + e) =
+            if constexpr (SAVE) *reinterpret_cast<uint2*>(Hs + (size_t)bh * (NT + 1) * KD * KD + (size_t)NT * KD * KD + e) =
                 make_uint2(pk2(acc[tp][0], acc[tp][1]), pk2(acc[tp][2], acc[tp][3]));
             if (hT)
                 *reinterpret_cast<float4*>(hT + sbase + e) =
                     make_float4(acc[tp][0], acc[tp][1], acc[tp][2], acc[tp][3]);
         }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// a few tokens without a backward (decoding)
+// ---------------------------------------------------------------------------
+// The recurrence itself, in fp32: one 256-thread workgroup per (b,h), thread (ig, jg) = (tid >> 4,
+// tid & 15) holding the state rows 4 ig.. x columns 4 jg.. in registers, read and written once
+// (row pieces of 256 contiguous bytes).  Per token the 16 row groups' sums of o are combined by
+// row swaps and one LDS exchange (double-buffered: one barrier a token), the next token's
+// operands loaded ahead.  Bound by the state's 32 KB a sequence at large B*H and by latency
+// below; a walk spends a whole chunk's operand tiles on any T <= 64.  Walk -> tokens: one token of
+// 8 x 32 heads 8.3 -> 3.7 us, of 64 x 64 heads 94 -> 21.5 us (6.4 TB/s); 8 tokens of 8 x 32
+// heads 8.4 -> 7.3, of 8 heads 6.8 -> 6.4, of 64 x 32 heads 50 -> 24 (the walks run in rounds of
+// 256 there): hence the bounds.
+#define TOK_THR 256
+inline bool few_tokens(int64_t BH, int64_t T) { return T > 0 && T <= (BH < 1024 ? 8 : 16); }
+template <bool SEQ>
+__global__ void __launch_bounds__(TOK_THR)
+wkv6_fwd_tokens(const uint16_t* __restrict__ r, const uint16_t* __restrict__ k,
+                const uint16_t* __restrict__ v, const uint16_t* __restrict__ w,
+                const void* __restrict__ u, int u_dtype, const float* __restrict__ h0,
+                uint16_t* __restrict__ o, float* __restrict__ hT, float scale, int B, int H, int T) {
+    __shared__ __attribute__((aligned(16))) float red[2][TOK_THR / 64][KD];
+    const int bh = blockIdx.x, h = bh % H, tid = threadIdx.x, wv = tid >> 6;
+    const int i0 = 4 * (tid >> 4), j0 = 4 * (tid & 15);
+    const size_t rs = tok_rs<SEQ>(B, H), base = tok_base<SEQ>(bh, 0, B, H, T), e = (size_t)bh * KD * KD + i0 * KD + j0;
+    struct Tok { uint2 r, k, v, w; };
+    auto load = [&](int t) {
+        const size_t b = base + (size_t)t * rs;
+        return Tok{*reinterpret_cast<const uint2*>(r + b + i0), *reinterpret_cast<const uint2*>(k + b + i0),
+                   *reinterpret_cast<const uint2*>(v + b + j0), *reinterpret_cast<const uint2*>(w + b + i0)};
+    };
+    Tok nx = load(0);
+    f32x4 S[4] = {};
+    if (h0) {
+#pragma unroll
+        for (int a = 0; a < 4; ++a) S[a] = *reinterpret_cast<const f32x4*>(h0 + e + a * KD);
+    }
+    float uf[4];
+#pragma unroll
+    for (int a = 0; a < 4; ++a) uf[a] = load_u(u, u_dtype, h * KD + i0 + a);
+    for (int t = 0; t < T; ++t) {
+        const Tok x = nx;
+        nx = load(min(t + 1, T - 1));
+        float rf[4], kf[4], vf[4], wf[4];
+        unpack4(x.r, rf);
+        unpack4(x.k, kf);
+        unpack4(x.v, vf);
+        unpack4(x.w, wf);
+        f32x4 acc = {};
+        const f32x4 vv = {vf[0], vf[1], vf[2], vf[3]};
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+            const float wl = SEQ ? -ex2(wf[a] * RW_L2E) : wf[a];
+            const f32x4 kv = kf[a] * vv;
+            acc += rf[a] * (S[a] + uf[a] * kv);
+            S[a] = ex2(fmaxf(wl, W_MIN) * RW_L2E) * S[a] + kv;
+        }
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+            const RowSums rsum = row_sums(acc[b]);
+            acc[b] = rsum.lo + rsum.hi;
+        }
+        if ((tid & 63) < 16) *reinterpret_cast<f32x4*>(&red[t & 1][wv][j0]) = acc;
+        __syncthreads();
+        if (tid < 16) {
+            f32x4 y = {};
+#pragma unroll
+            for (int q = 0; q < TOK_THR / 64; ++q) y += *reinterpret_cast<const f32x4*>(&red[t & 1][q][j0]);
+            *reinterpret_cast<uint2*>(o + ((size_t)bh * T + t) * KD + j0) =
+                make_uint2(pk2(scale * y[0], scale * y[1]), pk2(scale * y[2], scale * y[3]));
+        }
+    }
+    if (hT) {
+#pragma unroll
+        for (int a = 0; a < 4; ++a) *reinterpret_cast<f32x4*>(hT + e + a * KD) = S[a];
     }
 }
 
@@ -2783,10 +2863,14 @@ int lds_attributes(hipStream_t stream) {
             size_t bytes;
         };
         const Lds list[] = {
-            {reinterpret_cast<const void*>(wkv6_fwd_walk<false, false>), sizeof(WalkSmem)},
-            {reinterpret_cast<const void*>(wkv6_fwd_walk<true, false>), sizeof(WalkSmem)},
-            {reinterpret_cast<const void*>(wkv6_fwd_walk<false, true>), WALK_PRE_LDS},
-            {reinterpret_cast<const void*>(wkv6_fwd_walk<true, true>), WALK_PRE_LDS},
+            {reinterpret_cast<const void*>(wkv6_fwd_walk<false, false, false>), sizeof(WalkSmem)},
+            {reinterpret_cast<const void*>(wkv6_fwd_walk<false, false, true>), sizeof(WalkSmem)},
+            {reinterpret_cast<const void*>(wkv6_fwd_walk<false, true, false>), WALK_PRE_LDS},
+            {reinterpret_cast<const void*>(wkv6_fwd_walk<false, true, true>), WALK_PRE_LDS},
+            {reinterpret_cast<const void*>(wkv6_fwd_walk<true, false, false>), sizeof(WalkSmem)},
+            {reinterpret_cast<const void*>(wkv6_fwd_walk<true, false, true>), sizeof(WalkSmem)},
+            {reinterpret_cast<const void*>(wkv6_fwd_walk<true, true, false>), WALK_PRE_LDS},
+            {reinterpret_cast<const void*>(wkv6_fwd_walk<true, true, true>), WALK_PRE_LDS},
             {reinterpret_cast<const void*>(wkv6_bwd_loop<false, false>), sizeof(LoopSmem)},
             {reinterpret_cast<const void*>(wkv6_bwd_loop<true, false>), sizeof(LoopSmem)},
             {reinterpret_cast<const void*>(wkv6_bwd_loop<false, true>), sizeof(LoopSmem)},
@@ -2808,11 +2892,12 @@ template <bool SEQ>
 int wkv_fwd_impl(const void* r, const void* k, const void* v, const void* w, const void* u,
                  int u_dtype, const float* h0, void* o, float* hT, void* saved, void* workspace,
                  int64_t B, int64_t H, int64_t T, int64_t K, int64_t V, float scale,
-                 void* stream, void* const* phase_events, int64_t max_pieces = PIECE_TARGET) {
+                 void* stream, void* const* phase_events, int64_t max_pieces = PIECE_TARGET,
+                 bool infer = false) {
     int st = check_shape(B, H, T, K, V);
     if (st != RWKV6_OK) return st;
     if (u_dtype != RWKV6_F32 && u_dtype != RWKV6_BF16) return RWKV6_ERR_INVALID_ARG;
-    if (!u || !saved || (T > 0 && (!r || !k || !v || !w || !o || !workspace)))
+    if (!u || infer != !saved || (T > 0 && (!r || !k || !v || !w || !o || !workspace)))
         return RWKV6_ERR_INVALID_ARG;
     if (!al16(r) || !al16(k) || !al16(v) || !al16(w) || !al16(u) || !al16(o) || !al16(saved) ||
         !al16(workspace) || (h0 && !al16(h0)) || (hT && !al16(hT)))
@@ -2828,6 +2913,12 @@ int wkv_fwd_impl(const void* r, const void* k, const void* v, const void* w, con
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     const int64_t NT = nchunks(T);
     const int BH = (int)(B * H);
+    if (infer && few_tokens(BH, T)) {
+        hipLaunchKernelGGL(wkv6_fwd_tokens<SEQ>, dim3((unsigned)BH), dim3(TOK_THR), 0, s, (const uint16_t*)r,
+                           (const uint16_t*)k, (const uint16_t*)v, (const uint16_t*)w, u, u_dtype, h0,
+                           (uint16_t*)o, hT, scale, (int)B, (int)H, (int)T);
+        return launch_status();
+    }
     const WalkPlan plan = fwd_walk_plan(BH, NT);
     const int P = plan.P;
     const Pieces pc = prepass_pieces(BH, NT, P, max_pieces);
@@ -2852,7 +2943,8 @@ int wkv_fwd_impl(const void* r, const void* k, const void* v, const void* w, con
     mark(phase_events, 2, s);
     mark(phase_events, 3, s);
     mark(phase_events, 4, s);
-    auto walk = plan.pre ? wkv6_fwd_walk<SEQ, true> : wkv6_fwd_walk<SEQ, false>;
+    auto walk = saved ? (plan.pre ? wkv6_fwd_walk<SEQ, true, true> : wkv6_fwd_walk<SEQ, false, true>)
+                      : (plan.pre ? wkv6_fwd_walk<SEQ, true, false> : wkv6_fwd_walk<SEQ, false, false>);
     hipLaunchKernelGGL(walk, dim3((unsigned)(BH * P)), dim3(NTHR_W),
                        plan.pre ? WALK_PRE_LDS : sizeof(WalkSmem), s, (const uint16_t*)r, (const uint16_t*)k,
                        (const uint16_t*)v, (const uint16_t*)w, u, u_dtype, h0, (uint16_t*)o, Hs,
@@ -3072,6 +3164,14 @@ int rwkv6_wkv_bwd(const void* r, const void* k, const void* v, const void* w, co
                   void* stream) {
     return wkv_bwd_impl<false>(r, k, v, w, u, u_dtype, dO, dhT, saved, dr, dk, dv, dw, du, dh0,
                                workspace, B, H, T, K, V, scale, stream, nullptr);
+}
+
+int rwkv6_wkv_infer(const void* r, const void* k, const void* v, const void* w, const void* u,
+                    int u_dtype, const float* h0, void* o, float* hT, void* workspace, int seq_first,
+                    int64_t B, int64_t H, int64_t T, int64_t K, int64_t V, float scale, void* stream) {
+    auto fn = seq_first ? wkv_fwd_impl<true> : wkv_fwd_impl<false>;
+    return fn(r, k, v, w, u, u_dtype, h0, o, hT, nullptr, workspace, B, H, T, K, V, scale, stream, nullptr,
+              PIECE_TARGET, true);
 }
 
 int rwkv6_wkv_fwd_seqfirst(const void* r, const void* k, const void* v, const void* decay,

@@ -356,3 +356,33 @@ def test_wkv_plans(pkg, shape, plan, seq_first):
     ref = run_oracle(x, 1.0, True, True)
     ref["dw"] = ref["dw"] * _n(x["w"])
     _compare(got, ref, ["o", "hT", "dr", "dk", "dv", "dw", "du", "dh0"])
+
+
+# without gradients: the token kernel (T <= 8; 16 from 1024 sequences on), the walks without
+# chunk states past it (one chunk, a ragged second one, segments that form their own starts, the
+# pre-pass).  o and hT of the recurrence in fp32 carry o's bf16 rounding alone (2^-9), the walks'
+# the bars of the forward.
+@pytest.mark.parametrize("shape", [(1, 1, 1), (3, 2, 2), (2, 3, 7), (2, 2, 8), (2, 2, 9), (16, 64, 1), (16, 64, 16),
+                                   (16, 64, 17), (1, 2, 64), (1, 2, 65), (2, 8, 500), (1, 32, 2050)])
+@pytest.mark.parametrize("state", [False, True])
+def test_wkv_without_gradients(pkg, shape, state):
+    B, H, T = shape
+    x = _inputs(B, H, T, seed=B + H + T, w_hi=3.0)                # some tokens past the decay floor
+    scale = 0.5 if state else 1.0
+    dev = torch.device("cuda:0")
+    r, k, v, w, u, h0 = (x[n].to(dev) for n in ("r", "k", "v", "w", "u", "h0"))
+    ref = run_oracle(x, scale, state, False)
+    with torch.no_grad():
+        o, hT = pkg.fused_recurrent_rwkv6(r, k, v, w, u, scale=scale, initial_state=h0 if state else None,
+                                          output_final_state=True)
+        o2, none = pkg.chunk_rwkv6(r, k, v, w, u, scale=scale, initial_state=h0 if state else None)
+    assert none is None and torch.equal(o, o2) and not o.requires_grad
+    _compare(dict(o=_n(o), hT=_n(hT)), ref, ["o", "hT"])
+    tb = lambda t: t.permute(2, 0, 1, 3).reshape(T, B, H * 64).contiguous()
+    decay = torch.log(-x["w"].float()).to(torch.bfloat16)
+    x["w"] = -torch.exp(decay.float())
+    ref = run_oracle(x, scale, state, False)
+    with torch.no_grad():
+        o, hT = pkg.wkv6_seqfirst(tb(r), tb(k), tb(v), tb(decay.to(dev)), u, H, scale=scale,
+                                  initial_state=h0 if state else None, output_final_state=True)
+    _compare(dict(o=_n(o), hT=_n(hT)), ref, ["o", "hT"])
