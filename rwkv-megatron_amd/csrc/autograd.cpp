@@ -425,18 +425,24 @@ Tensor sum_partials(const Tensor& part, at::ScalarType dt) {
 
 // dW = dy^T x for dy [N, O], x [N, I] (N = tokens), fp32-accumulated.  A projection's weight
 // gradient has a small output (O x I, e.g. 2048 x 2048 = 64 tiles of 256 x 256) and a long
-// reduction (16 K tokens): one GEMM occupies a quarter of the 256 CUs.  The tokens are split into
-// s chunks (s doubles while the tile count stays below 512, at most 4: at 16 K tokens a 2048 x
-// 2048 dW takes 155 us with s = 4 against 170 us with s = 8, whose partial sum reads twice the
-// bytes), the chunks run as one batched GEMM with fp32 outputs, and the partials are summed in a
-// fixed order.
+// reduction (16 K tokens): one GEMM occupies a quarter of the 256 CUs.  The tokens are split into s
+// chunks that run as one batched GEMM with fp32 outputs, summed in a fixed order, where that is
+// faster than the s partial sums cost: s doubles up to 4 while the tiles of all chunks are below
+// the CU count and a chunk keeps 4096 tokens (2560 for an output of a few tiles, which leaves more
+// CUs idle).  Measured on MI355X, us for s = 1, 2, 4: 2048 x 2048 of 16384 tokens 163, 140, 136, of
+// 8192 tokens 102, 88, 91, of 4096 tokens 44, 49, 56; 7168 x 2048 of 8192 tokens 297, 258, 302, of
+// 4096 tokens 140, 168, 206; 1024 x 1024 of 8192 tokens 55, 39, 36.  One chunk writes dt directly (a
+// parameter wider than bf16 gets the fp32 accumulator).
 Tensor splitk_wgrad(const Tensor& dy, const Tensor& x, at::ScalarType dt) {
     const int64_t N = dy.size(0), O = dy.size(1), I = x.size(1), tiles = (O + 255) / 256 * ((I + 255) / 256);
+    const int64_t chunk = tiles > 32 ? 4096 : 2560;
     int64_t s = 1;
-    while (s < 4 && tiles * s < 512 && N % (2 * s) == 0) s *= 2;
-    if (s == 1) return cast(at::mm(dy.t(), x), dt);
+    while (s < 4 && tiles * s < 256 && N % (2 * s) == 0 && N / (2 * s) >= chunk) s *= 2;
+    if (s == 1 && (!dy.is_cuda() || dt == dy.scalar_type() || dy.scalar_type() != at::kBFloat16 || N == 0))
+        return cast(at::mm(dy.t(), x), dt);
     TORCH_CHECK_TYPE(dy.is_cuda(), "split weight gradients run on the GPU");
-    return sum_partials(at::bmm(dy.view({s, N / s, O}).transpose(1, 2), x.view({s, N / s, I}), at::kFloat), dt);
+    const Tensor part = at::bmm(dy.view({s, N / s, O}).transpose(1, 2), x.view({s, N / s, I}), at::kFloat);
+    return s == 1 ? cast(part.view({O, I}), dt) : sum_partials(part, dt);
 }
 
 struct Linear : torch::autograd::Function<Linear> {
