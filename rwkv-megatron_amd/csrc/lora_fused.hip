@@ -21,9 +21,10 @@
 // all tokens of a channel.  Reading d_out and x twice (12 x 2C bytes a token) and recomputing
 // m = neck W_up costs less than passing dm ([5,N,C]), the two lerp sums, xxx and d_xxx through
 // HBM between a kernel per step and the library's batched GEMMs of 32 columns.  Measured at N =
-// 16384, C = 2048, forward and backward: the token shift 721 -> 414 us (18 -> 5 launches), the
-// decay 412 -> 182 us (16 -> 5); the general path (other ranks) is in timemix.py.
+// 16384, C = 2048, forward and backward: the token shift 718 -> 400 us (18 -> 5 launches), the
+// decay 391 -> 127 us (16 -> 5); the general path (other ranks) is in timemix.py.
 #include <algorithm>
+#include <utility>
 
 #include "common.h"
 #include "../../include/rwkv6_amd.h"
@@ -87,21 +88,21 @@ __device__ __forceinline__ void p_f32(const PRaw& r, int dtype, float* f) {
 }  // namespace
 
 // neck[n][r] = tanh(sum_c xxx[n][c] W_down[c][r]), xxx = x + (shift(x) - x) maa rounded to bf16
-// (LERP) or x.  Workgroup = 64 token rows x all ER columns, 64 channels a step through double-
+// (LERP) or x.  Workgroup = TT token rows x all ER columns, 64 channels a step through double-
 // buffered LDS tiles (one barrier a step), the loads of two steps ahead in registers.  The
 // product is formed transposed (W_down^T as the A operand), so a lane ends with four adjacent
 // columns of one token.  Wave (tt, hh) takes tokens 16 tt.. and the column tiles 2i + hh.
-template <int ER, bool LERP, bool WF32>
-__global__ void __launch_bounds__(LF_THR)
+template <int ER, bool LERP, bool WF32, int TT>
+__global__ void __launch_bounds__(8 * TT)
 rwkv6_lora_down_kernel(const uint16_t* __restrict__ x, const void* __restrict__ maa, int mdt,
                        const void* __restrict__ wd, uint16_t* __restrict__ neck, int64_t N,
                        int64_t B, int64_t C) {
-    constexpr int WS = ER + 8, NP = LF_TT * ER / 8, NPT = (NP + LF_THR - 1) / LF_THR, NA = ER / 32;
-    __shared__ __attribute__((aligned(16))) uint16_t xs[2][LF_TT][LF_TS];
-    __shared__ __attribute__((aligned(16))) uint16_t ws[2][LF_TT][WS];
+    constexpr int WS = ER + 8, THR = 8 * TT, NP = 64 * ER / 8, NPT = (NP + THR - 1) / THR, NA = ER / 32;
+    __shared__ __attribute__((aligned(16))) uint16_t xs[2][TT][LF_TS];
+    __shared__ __attribute__((aligned(16))) uint16_t ws[2][64][WS];
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, L = lane & 15, q = lane >> 4;
-    const int tt = wv & 3, hh = wv >> 2, row = tid >> 3, cg = tid & 7;
-    const int64_t n0 = (int64_t)blockIdx.x * LF_TT, n = n0 + row < N ? n0 + row : N - 1;
+    const int tt = wv % (TT / 16), hh = wv / (TT / 16), row = tid >> 3, cg = tid & 7;
+    const int64_t n0 = (int64_t)blockIdx.x * TT, n = n0 + row < N ? n0 + row : N - 1;
     const uint16_t* xrow = x + n * C + 8 * cg;
     const uint16_t* prow = x + (n >= B ? n - B : n) * C + 8 * cg;
     const float keep = n >= B ? 1.f : 0.f;
@@ -115,7 +116,7 @@ rwkv6_lora_down_kernel(const uint16_t* __restrict__ x, const void* __restrict__ 
         }
 #pragma unroll
         for (int i = 0; i < NPT; ++i)          // the tile's 64 rows are contiguous; a piece past
-            s.w[i] = w_load<WF32>(wd, (int64_t)64 * k * ER + 8 * min(tid + LF_THR * i, NP - 1));  // the end repeats the last
+            s.w[i] = w_load<WF32>(wd, (int64_t)64 * k * ER + 8 * min(tid + THR * i, NP - 1));  // the end repeats the last
     };
     f32x4 acc[NA] = {};
     auto step = [&](Step& s, int k) {
@@ -134,7 +135,7 @@ rwkv6_lora_down_kernel(const uint16_t* __restrict__ x, const void* __restrict__ 
         *reinterpret_cast<uint4*>(&xt[row][8 * cg]) = xq;
 #pragma unroll
         for (int i = 0; i < NPT; ++i) {
-            const int p = min(tid + LF_THR * i, NP - 1);
+            const int p = min(tid + THR * i, NP - 1);
             *reinterpret_cast<uint4*>(&wt[p / (ER / 8)][8 * (p % (ER / 8))]) = w_bf16<WF32>(s.w[i]);
         }
         __syncthreads();
@@ -165,24 +166,25 @@ rwkv6_lora_down_kernel(const uint16_t* __restrict__ x, const void* __restrict__ 
 
 // d_pre[n][e R + r] = (sum_c dm_e[n][c] W_up[e][r][c]) (1 - neck^2), dm_e = d_out_e (shift(x) -
 // x) rounded to bf16 (LERP; the MFMA operand the weight gradient uses too) or d_out_e.
-// Workgroup = 64 token rows x all channels, as the down kernel; per step the dm tiles of all
-// mixes and W_up's 64 columns go to LDS.  Bound by reading d_out and x.
-template <int E, int R, bool LERP>
+// Workgroup = TT token rows x all channels, as the down kernel; per step the dm tiles of all
+// mixes and W_up's 64 columns go to LDS.  Bound by reading d_out and x: the mixes load two steps
+// ahead (N = 16384, C = 2048: 105 -> 90 us against one step), the decay's smaller step four.
+template <int E, int R, int TT>
 struct DpreSmem {
-    uint16_t dm[2][E][LF_TT][LF_TS];
+    uint16_t dm[2][E][TT][LF_TS];
     uint16_t w[2][E * R][LF_TS];
 };
-template <int E, int R, bool LERP, bool WF32, int DEPTH>
-__global__ void __launch_bounds__(LF_THR)
+template <int E, int R, bool LERP, bool WF32, int DEPTH, int TT>
+__global__ void __launch_bounds__(8 * TT)
 rwkv6_lora_dpre_kernel(const uint16_t* __restrict__ x, InPtrs<E> dout,
                        const uint16_t* __restrict__ neck, const void* __restrict__ wup,
                        uint16_t* __restrict__ dpre, int64_t N, int64_t B, int64_t C) {
-    constexpr int ER = E * R, NP = ER * 8, NPT = (NP + LF_THR - 1) / LF_THR, NA = ER / 32;
+    constexpr int ER = E * R, THR = 8 * TT, NP = ER * 8, NPT = (NP + THR - 1) / THR, NA = ER / 32;
     extern __shared__ __attribute__((aligned(16))) unsigned char lf_smem[];
-    DpreSmem<E, R, LERP>& sm = *reinterpret_cast<DpreSmem<E, R, LERP>*>(lf_smem);
+    DpreSmem<E, R, TT>& sm = *reinterpret_cast<DpreSmem<E, R, TT>*>(lf_smem);
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, L = lane & 15, q = lane >> 4;
-    const int tt = wv & 3, hh = wv >> 2, row = tid >> 3, cg = tid & 7;
-    const int64_t n0 = (int64_t)blockIdx.x * LF_TT, n = n0 + row < N ? n0 + row : N - 1;
+    const int tt = wv % (TT / 16), hh = wv / (TT / 16), row = tid >> 3, cg = tid & 7;
+    const int64_t n0 = (int64_t)blockIdx.x * TT, n = n0 + row < N ? n0 + row : N - 1;
     const int64_t xo = n * C + 8 * cg, po = (n >= B ? n - B : n) * C + 8 * cg;
     const float keep = n >= B ? 1.f : 0.f;
     const int nk = (int)(C / 64);
@@ -190,7 +192,7 @@ rwkv6_lora_dpre_kernel(const uint16_t* __restrict__ x, InPtrs<E> dout,
     auto load = [&](Step& s, int k) {
 #pragma unroll
         for (int i = 0; i < NPT; ++i) {
-            const int p = min(tid + LF_THR * i, NP - 1);
+            const int p = min(tid + THR * i, NP - 1);
             s.w[i] = w_load<WF32>(wup, (int64_t)(p >> 3) * C + 64 * k + 8 * (p & 7));
         }
         if (LERP) {
@@ -205,7 +207,7 @@ rwkv6_lora_dpre_kernel(const uint16_t* __restrict__ x, InPtrs<E> dout,
         const int bf = k & 1;
 #pragma unroll
         for (int i = 0; i < NPT; ++i) {
-            const int p = min(tid + LF_THR * i, NP - 1);
+            const int p = min(tid + THR * i, NP - 1);
             *reinterpret_cast<uint4*>(&sm.w[bf][p >> 3][8 * (p & 7)]) = w_bf16<WF32>(s.w[i]);
         }
         if (LERP) {
@@ -237,18 +239,20 @@ rwkv6_lora_dpre_kernel(const uint16_t* __restrict__ x, InPtrs<E> dout,
                 acc[i] = mfma32(ld_bf16x8(&sm.w[bf][16 * rt + L][32 * ks + 8 * q]), b, acc[i]);
             }
     };
-    static_assert(DEPTH == 1 || DEPTH == 4, "ring of one or four steps");
+    static_assert(DEPTH == 1 || DEPTH == 2 || DEPTH == 4, "ring of one, two or four steps");
     Step s0, s1, s2, s3;
     load(s0, 0);
+    if constexpr (DEPTH >= 2) load(s1, min(1, nk - 1));
     if constexpr (DEPTH == 4) {
-        load(s1, min(1, nk - 1));
         load(s2, min(2, nk - 1));
         load(s3, min(3, nk - 1));
     }
     for (int k = 0; k < nk; k += DEPTH) {
         step(s0, k);
-        if constexpr (DEPTH == 4) {
+        if constexpr (DEPTH >= 2) {
             if (k + 1 < nk) step(s1, k + 1);
+        }
+        if constexpr (DEPTH == 4) {
             if (k + 2 < nk) step(s2, k + 2);
             if (k + 3 < nk) step(s3, k + 3);
         }
@@ -292,7 +296,7 @@ struct GradsSmem {
 };
 static_assert(sizeof(GradsSmem<LF_E_MIX, LF_R_MIX, true>) <= 160 * 1024, "one workgroup per CU");
 static_assert(2 * sizeof(GradsSmem<1, LF_R_DECAY, false>) <= 160 * 1024, "two workgroups per CU");
-static_assert(sizeof(DpreSmem<LF_E_MIX, LF_R_MIX, true>) <= 160 * 1024, "one workgroup per CU");
+static_assert(sizeof(DpreSmem<LF_E_MIX, LF_R_MIX, 64>) <= 160 * 1024, "one workgroup per CU");
 // partial parameter gradients of one workgroup range: dW_up [ER][C], dW_down [C][ER], d_bias
 // [E][C], d_maa [C] (LERP)
 __host__ __device__ constexpr int64_t lf_cols(int64_t E, int64_t R, int64_t C, bool lerp) {
@@ -575,6 +579,12 @@ inline bool lf_supported(int64_t B, int64_t C, int64_t E, int64_t R, bool lerp) 
     return (lerp ? E == LF_E_MIX && R == LF_R_MIX : E == 1 && R == LF_R_DECAY) && C <= (1 << 23) &&
            B <= (1 << 23) / C;
 }
+// Token rows of a workgroup of the down and d_pre kernels.  Each workgroup reads the whole weight,
+// so the mixes' 64 rows halve that traffic once 64 rows a workgroup still give half the CUs one
+// (N = 16384, C = 2048: d_pre 88 against 106 us, down 42 against 45.5); below that, and for the
+// decay's smaller weight, 32 rows spread a short walk over twice the CUs (N = 1024, C = 512:
+// mixes 18 -> 12.4 and 13.4 -> 10.9 us, decay 6.9 -> 5.0 and 9.1 -> 5.5).
+inline int lf_tile(int64_t N, bool lerp) { return lerp && N > 8192 ? 64 : 32; }
 // Tiles, tiles a range and ranges of the gradient kernel.  The time is the rounds of
 // workgroups over the device times the tiles of a range; fewer ranges (less partial traffic)
 // win ties.  `slots`: workgroups the device holds at once (LDS: one LERP workgroup of 157 KB a
@@ -609,15 +619,17 @@ int rwkv6_lora_down_fwd(const void* x, const void* maa, int maa_dtype, const voi
     if (!x || !w_down || !neck) return RWKV6_ERR_INVALID_ARG;
     if (!al16(x) || !al16(maa) || !al16(w_down) || !al16(neck)) return RWKV6_ERR_ALIGNMENT;
     const int64_t N = T * B;
-    if ((N + LF_TT - 1) / LF_TT > 0x7fffffff) return RWKV6_ERR_UNSUPPORTED;
+    if (N > ((int64_t)1 << 36)) return RWKV6_ERR_UNSUPPORTED;          // the grid's range
     if (any_alias({{neck, (size_t)(N * E * R) * 2}},
                   {{x, (size_t)(N * C) * 2}, {maa, (size_t)C * param_bytes(maa_dtype)},
                    {w_down, (size_t)(C * E * R) * param_bytes(w_dtype)}}))
         return RWKV6_ERR_INVALID_ARG;
     constexpr int MIX = LF_E_MIX * LF_R_MIX, DEC = LF_R_DECAY;
-    auto kern = lerp ? (f32 ? rwkv6_lora_down_kernel<MIX, true, true> : rwkv6_lora_down_kernel<MIX, true, false>)
-                     : (f32 ? rwkv6_lora_down_kernel<DEC, false, true> : rwkv6_lora_down_kernel<DEC, false, false>);
-    hipLaunchKernelGGL(kern, dim3((unsigned)((N + LF_TT - 1) / LF_TT)), dim3(LF_THR), 0,
+    const int tt = lf_tile(N, lerp);
+    auto kern = !lerp ? (f32 ? rwkv6_lora_down_kernel<DEC, false, true, 32> : rwkv6_lora_down_kernel<DEC, false, false, 32>)
+                : tt == 64 ? (f32 ? rwkv6_lora_down_kernel<MIX, true, true, 64> : rwkv6_lora_down_kernel<MIX, true, false, 64>)
+                           : (f32 ? rwkv6_lora_down_kernel<MIX, true, true, 32> : rwkv6_lora_down_kernel<MIX, true, false, 32>);
+    hipLaunchKernelGGL(kern, dim3((unsigned)((N + tt - 1) / tt)), dim3(8 * tt), 0,
                        reinterpret_cast<hipStream_t>(stream), (const uint16_t*)x, maa, maa_dtype, w_down,
                        (uint16_t*)neck, N, B, C);
     return launch_status();
@@ -644,22 +656,28 @@ int lora_bwd_launch(const uint16_t* x, const void* maa, int mdt, const InPtrs<E>
     uint16_t* dpre = reinterpret_cast<uint16_t*>(workspace);
     float* part = reinterpret_cast<float*>(reinterpret_cast<char*>(workspace) + lf_round((size_t)(N * E * R) * 2));
     if (N > 0) {
-        auto kp = rwkv6_lora_dpre_kernel<E, R, LERP, WF32, DEPTH>;
+        const int tt = lf_tile(N, LERP);
+        auto kp64 = rwkv6_lora_dpre_kernel<E, R, LERP, WF32, DEPTH, LERP ? 64 : 32>;
+        auto kp32 = rwkv6_lora_dpre_kernel<E, R, LERP, WF32, DEPTH, 32>;
         auto kg = rwkv6_lora_grads_kernel<E, R, LERP, WF32>;
         static DeviceOnce once[kMaxDevices];
         int dev = 0, cur = 0, st = stream_device(s, &dev, &cur);
         if (st != RWKV6_OK) return st;
         st = device_once(once[dev], dev, cur, [&] {
-            hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kp), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                               (int)sizeof(DpreSmem<E, R, LERP>));
-            return e != hipSuccess ? e
-                                   : hipFuncSetAttribute(reinterpret_cast<const void*>(kg),
-                                                         hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                         (int)sizeof(GradsSmem<E, R, LERP>));
+            const std::pair<const void*, size_t> list[] = {
+                {reinterpret_cast<const void*>(kp64), sizeof(DpreSmem<E, R, LERP ? 64 : 32>)},
+                {reinterpret_cast<const void*>(kp32), sizeof(DpreSmem<E, R, 32>)},
+                {reinterpret_cast<const void*>(kg), sizeof(GradsSmem<E, R, LERP>)}};
+            hipError_t e = hipSuccess;
+            for (const auto& x : list)
+                if (e == hipSuccess)
+                    e = hipFuncSetAttribute(x.first, hipFuncAttributeMaxDynamicSharedMemorySize, (int)x.second);
+            return e;
         });
         if (st != RWKV6_OK) return st;
-        hipLaunchKernelGGL(kp, dim3((unsigned)((N + LF_TT - 1) / LF_TT)), dim3(LF_THR), sizeof(DpreSmem<E, R, LERP>),
-                           s, x, dout, neck, wup, dpre, N, B, C);
+        hipLaunchKernelGGL(tt == 64 ? kp64 : kp32, dim3((unsigned)((N + tt - 1) / tt)), dim3(8 * tt),
+                           tt == 64 ? sizeof(DpreSmem<E, R, 64>) : sizeof(DpreSmem<E, R, 32>), s, x, dout, neck, wup,
+                           dpre, N, B, C);
         hipLaunchKernelGGL(kg, dim3((unsigned)(8 * ((p.np + 7) / 8) * (C / 64))), dim3(LF_THR),
                            sizeof(GradsSmem<E, R, LERP>), s, x, maa, mdt, dout, neck, (const uint16_t*)dpre, wup, wd,
                            bias, bdt, dx, part, LERP ? T : N, LERP ? B : (int64_t)1, C, p.ntiles, p.tpr, p.nr, p.np);
@@ -719,7 +737,7 @@ int rwkv6_lora_bwd(const void* x, const void* maa, int maa_dtype, const void* co
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     const uint16_t *xp = (const uint16_t*)x, *np = (const uint16_t*)neck;
     if (lerp) {
-        auto go = f32 ? lora_bwd_launch<LF_E_MIX, LF_R_MIX, true, true, 1> : lora_bwd_launch<LF_E_MIX, LF_R_MIX, true, false, 1>;
+        auto go = f32 ? lora_bwd_launch<LF_E_MIX, LF_R_MIX, true, true, 2> : lora_bwd_launch<LF_E_MIX, LF_R_MIX, true, false, 2>;
         return go(xp, maa, maa_dtype, dm, np, w_down, w_up, bias, bias_dtype, (uint16_t*)dx, o, workspace, T, B, C, s);
     }
     InPtrs<1> d1;

@@ -376,7 +376,9 @@ def _bottleneck_run(pkg, form, leaves, dy, general=False):
     (65, 1, 64, torch.bfloat16, torch.float32, torch.float32),
     (127, 3, 64, torch.float32, torch.float32, torch.float32),
     (128, 1, 64, torch.float16, torch.bfloat16, torch.float16),
-    (1009, 2, 512, torch.bfloat16, torch.bfloat16, torch.bfloat16)])
+    (1009, 2, 512, torch.bfloat16, torch.bfloat16, torch.bfloat16),
+    (4096, 2, 64, torch.bfloat16, torch.bfloat16, torch.bfloat16),      # the mixes' last 32-row tiles
+    (8193, 1, 64, torch.float32, torch.bfloat16, torch.float32)])       # 64-row tiles, one row over
 def test_bottleneck_kernels_match_the_general_path(pkg, form, T, B, C, wdt, udt, pdt):
     leaves, dy = _bottleneck_case(form, T, B, C, wdt, udt, pdt)
     got = _bottleneck_run(pkg, form, leaves, dy)
