@@ -257,6 +257,21 @@ int rwkv6_gn_gate_bwd(const void* o, int head_first, const void* g_pre, const vo
                       void* stream);
 
 /* ------------------------------------------------------------------------
+ * LayerNorm over the C channels of N bf16 rows (rwkv6_layer_specs.py:543-547), C a multiple of 8
+ * up to 4096 (else RWKV6_ERR_UNSUPPORTED).  gamma, beta: [C] in param_dtype; y: [N,C] bf16;
+ * mean, rstd: [N] f32 for the backward; gamma_copy: [C] f32, nullable: gamma as it was used.
+ * ---------------------------------------------------------------------- */
+int rwkv6_layer_norm_fwd(const void* x, const void* gamma, const void* beta, int param_dtype,
+                         float eps, void* y, float* mean, float* rstd, float* gamma_copy,
+                         int64_t N, int64_t C, void* stream);
+size_t rwkv6_layer_norm_bwd_workspace_bytes(int64_t N, int64_t C);
+/* dy [N,C] -> dx [N,C] bf16 and dgamma, dbeta [C] in param_dtype (both NULL: dx alone, no
+ * workspace). */
+int rwkv6_layer_norm_bwd(const void* x, const void* gamma, int gamma_dtype, const float* mean,
+                         const float* rstd, const void* dy, void* dx, void* dgamma, void* dbeta,
+                         int param_dtype, void* workspace, int64_t N, int64_t C, void* stream);
+
+/* ------------------------------------------------------------------------
  * Forward without a workspace argument.  No counterpart in the reference: for callers that
  * cannot allocate device memory (code under HIP graph capture, tight serving loops, harnesses
  * that forbid hipMalloc).  Same arguments and results as rwkv6_wkv_fwd minus `workspace`:

@@ -13,6 +13,10 @@
 // functions check their arguments and call these.
 #include <torch/extension.h>
 
+#include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/TracerMode.h>
+#include <ATen/autocast_mode.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 
 #include <cstring>
@@ -332,6 +336,83 @@ Tensor group_norm_gate(const Tensor& o, const OptTensor& g, const Tensor& gamma,
 }
 
 // ---------------------------------------------------------------------------------------
+// LayerNorm over the last dimension
+// ---------------------------------------------------------------------------------------
+struct LayerNorm : torch::autograd::Function<LayerNorm> {
+    static Tensor forward(AutogradContext* ctx, const Tensor& xi, const Tensor& gamma, const Tensor& beta, double eps,
+                          bool grad) {
+        const Tensor x = dense(xi);
+        const int64_t C = x.size(-1), N = x.numel() / C;
+        Param ga = param(gamma), be = param(beta);
+        if (ga.dt != be.dt) ga = {to_f32(gamma), RWKV6_F32}, be = {to_f32(beta), RWKV6_F32};
+        const Tensor y = at::empty_like(x), mean = empty({N}, at::kFloat, x), rstd = at::empty_like(mean);
+        // A bf16 gamma is saved itself.  Of any other the backward uses the values of this call, from
+        // the kernel's copy, so that an update of the parameter in between is not an error.
+        const Tensor copy = grad && gamma.scalar_type() != at::kBFloat16 ? empty({C}, at::kFloat, x) : Tensor();
+        check(rwkv6_layer_norm_fwd(ptr(x), ptr(ga.t), ptr(be.t), ga.dt, (float)eps, ptr(y), fptr(mean), fptr(rstd),
+                                   fptr(copy), N, C, stream_of(x)),
+              "rwkv6_layer_norm_fwd");
+        if (grad) {
+            ctx->save_for_backward({x, copy.defined() ? copy : gamma, mean, rstd});
+            if (copy.defined()) ctx->saved_data["gamma"] = gamma;
+            ctx->saved_data["beta"] = beta;
+        }
+        return y;
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list gr) {
+        const auto s = ctx->get_saved_variables();
+        const Tensor &x = s[0], &mean = s[2], &rstd = s[3];
+        const bool own = ctx->saved_data.count("gamma") == 0;       // gamma is the saved tensor itself
+        const Tensor gamma = own ? s[1] : ctx->saved_data["gamma"].toTensor(), beta = ctx->saved_data["beta"].toTensor();
+        const bool ng = ctx->needs_input_grad(1), nb = ctx->needs_input_grad(2);
+        const int64_t C = x.size(-1), N = x.numel() / C;
+        if (at::GradMode::is_enabled()) {
+            // a backward that is differentiated itself: torch's differentiable form, on the values used
+            const Tensor g = own ? gamma : gamma + (s[1].to(gamma.scalar_type()) - gamma).detach();
+            std::vector<int64_t> st(x.sizes().begin(), x.sizes().end());
+            st.back() = 1;
+            const auto [dx, dg, db] = at::native_layer_norm_backward(gr[0], x, {C}, mean.view(st), rstd.view(st),
+                                                                     g.to(x.scalar_type()), beta.to(x.scalar_type()),
+                                                                     {true, ng, nb});
+            return {dx, ng ? cast(dg, gamma.scalar_type()) : Tensor(), nb ? cast(db, beta.scalar_type()) : Tensor(), Tensor(), Tensor()};
+        }
+        const Param ga = param(s[1]);
+        const Tensor dy = to_bf16(gr[0]), dx = at::empty_like(x);
+        const int dt = grad_code(gamma) == grad_code(beta) ? grad_code(gamma) : RWKV6_F32;
+        const bool sums = ng || nb;
+        const Tensor dg = sums ? empty({C}, param_type(dt), x) : Tensor(), db = sums ? at::empty_like(dg) : Tensor();
+        const Tensor ws = sums ? bytes(rwkv6_layer_norm_bwd_workspace_bytes(N, C), x) : Tensor();
+        check(rwkv6_layer_norm_bwd(ptr(x), ptr(ga.t), ga.dt, fptr(mean), fptr(rstd), ptr(dy), ptr(dx), ptr(dg), ptr(db), dt,
+                                   ptr(ws), N, C, stream_of(x)),
+              "rwkv6_layer_norm_bwd");
+        return {dx, ng ? cast(dg, gamma.scalar_type()) : Tensor(), nb ? cast(db, beta.scalar_type()) : Tensor(), Tensor(), Tensor()};
+    }
+};
+// Whether an operator on these tensors is a plain call of its kernel: no autocast, transform,
+// tracing, forward-mode derivative or mode that wants to see it.
+bool plain(std::initializer_list<const Tensor*> ts) {
+    if (at::autocast::is_autocast_enabled(at::kCUDA) || c10::impl::dispatch_mode_enabled() ||
+        at::impl::torch_function_mode_enabled() || at::tracer::impl::is_dispatch_enabled() ||
+        c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode))
+        return false;
+    for (const Tensor* t : ts)
+        if (t->key_set().has(c10::DispatchKey::Python) || t->_fw_grad(0).defined()) return false;
+    return true;
+}
+// None when the kernels do not take the call: the caller runs torch's.
+py::object layer_norm(const Tensor& x, const OptTensor& gamma, const OptTensor& beta, double eps) {
+    if (!gamma || !beta || x.dim() < 1 || x.numel() == 0 || x.layout() != at::kStrided) return py::none();
+    const int64_t C = x.size(-1);
+    if (rwkv6_layer_norm_bwd_workspace_bytes(x.numel() / C, C) == 0) return py::none();
+    for (const Tensor* t : {&*gamma, &*beta})
+        if (t->sizes() != at::IntArrayRef({C}) || t->device() != x.device() ||
+            (t->scalar_type() != at::kBFloat16 && t->scalar_type() != at::kFloat && t->scalar_type() != at::kHalf))
+            return py::none();
+    if (!plain({&x, &*gamma, &*beta})) return py::none();
+    return py::cast(LayerNorm::apply(x, *gamma, *beta, eps, recorded({&x, &*gamma}, beta)));
+}
+
+// ---------------------------------------------------------------------------------------
 // channel mix
 // ---------------------------------------------------------------------------------------
 struct CmixLerp : torch::autograd::Function<CmixLerp> {
@@ -478,6 +559,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("token_shift_mix", torch::wrap_pybind_function(token_shift_mix));
     m.def("decay_lora", torch::wrap_pybind_function(decay_lora));
     m.def("group_norm_gate", torch::wrap_pybind_function(group_norm_gate));
+    m.def("layer_norm", torch::wrap_pybind_function(layer_norm));
     m.def("cmix_lerp", torch::wrap_pybind_function(cmix_lerp));
     m.def("relu_sq", torch::wrap_pybind_function(relu_sq));
     m.def("sigmoid_gate", torch::wrap_pybind_function(sigmoid_gate));

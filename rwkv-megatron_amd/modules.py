@@ -36,8 +36,8 @@ Deliberate differences, all documented in the reference's own terms:
     (l = 0) in every layer, and a checkpoint (from_rwkv_lm) sets the real values.
   * The decay bias keeps the reference's uniform(-1, 1) (:173-175) unless
     ``rwkv_lm_decay_init`` asks for RWKV-LM's ramp.
-  * LayerNorms and the output head cast their parameters to the activations' dtype, so fp32
-    parameters train with bf16 activations (the HIP kernels take bf16 activations).
+  * LayerNorms and the output head take fp32 parameters with bf16 activations (the HIP kernels
+    take bf16 activations; what runs through torch casts the parameters to them).
 """
 from __future__ import annotations
 
@@ -122,10 +122,16 @@ class _Linear(nn.Module):
 
 class LayerNorm(nn.LayerNorm):
     """Megatron's LayerNorm at TP = 1 (the layer spec's input_layernorm / pre_mlp_layernorm,
-    :543, :546, and the model's pre_norm / final_layernorm); the parameters are cast to the
-    activations' dtype, so fp32 parameters run with bf16 activations."""
+    :543, :546, and the model's pre_norm / final_layernorm).  bf16 activations on the GPU run on
+    the HIP kernels with the parameters as they are (rows of up to 4096 channels, a multiple of
+    8); anything else through torch with the parameters cast to the activations' dtype."""
 
     def forward(self, x):
+        if (type(x) is torch.Tensor and x.is_cuda and x.dtype == torch.bfloat16
+                and len(self.normalized_shape) == 1 and not torch.compiler.is_compiling()):
+            y = _lib.native().layer_norm(x, self.weight, self.bias, self.eps)
+            if y is not None:
+                return y
         return F.layer_norm(x, self.normalized_shape, self.weight.to(x.dtype), self.bias.to(x.dtype),
                             self.eps)
 
