@@ -257,6 +257,14 @@ int rwkv6_gn_gate_bwd(const void* o, int head_first, const void* g_pre, const vo
                       void* stream);
 
 /* ------------------------------------------------------------------------
+ * y [N,O] = x [N,I] W^T for few tokens: x, y bf16, W [O,I] fp32, rounded to bf16 inside and written
+ * to w_bf16 [O,I] where that is not NULL.  O a multiple of 4, I of 8, N > 0 (else
+ * RWKV6_ERR_UNSUPPORTED).
+ * ---------------------------------------------------------------------- */
+int rwkv6_linear_f32(const void* x, const float* w, void* y, void* w_bf16, int64_t N, int64_t O,
+                     int64_t I, void* stream);
+
+/* ------------------------------------------------------------------------
  * LayerNorm over the C channels of N bf16 rows (rwkv6_layer_specs.py:543-547), C a multiple of 8
  * up to 4096 (else RWKV6_ERR_UNSUPPORTED).  gamma, beta: [C] in param_dtype; y: [N,C] bf16;
  * mean, rstd: [N] f32 for the backward; gamma_copy: [C] f32, nullable: gamma as it was used.

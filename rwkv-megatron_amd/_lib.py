@@ -74,6 +74,7 @@ SIGNATURES = {
     "rwkv6_gn_gate_bwd_workspace_bytes": (ctypes.c_size_t, [_i64] * 4),
     "rwkv6_gn_gate_bwd": (_int, [_vp, _int, _vp, _vp, _vp, _int, _fp, _fp] + [_vp] * 5 + [_vp]
                           + [_i64] * 4 + [_vp]),
+    "rwkv6_linear_f32": (_int, [_vp, _fp, _vp, _vp] + [_i64] * 3 + [_vp]),
     "rwkv6_layer_norm_fwd": (_int, [_vp] * 3 + [_int, _f32, _vp, _fp, _fp, _fp] + [_i64] * 2 + [_vp]),
     "rwkv6_layer_norm_bwd_workspace_bytes": (ctypes.c_size_t, [_i64] * 2),
     "rwkv6_layer_norm_bwd": (_int, [_vp, _vp, _int, _fp, _fp] + [_vp] * 4 + [_int, _vp] + [_i64] * 2 + [_vp]),

@@ -526,8 +526,36 @@ Tensor splitk_wgrad(const Tensor& dy, const Tensor& x, at::ScalarType dt) {
     return s == 1 ? cast(part.view({O, I}), dt) : sum_partials(part, dt);
 }
 
+// Whether y = x W^T runs on the kernel that rounds an fp32 W inside instead of a cast and the library's
+// product: up to 2^30 multiplications (1024 tokens x 1024 x 1024: 12.1 us against 13.7; 1536: 16.5
+// against 14.5), 2048 inputs (a longer chain of steps: 1024 x 3584 of 64 tokens 18.5 and 20.1 us, of
+// 777 33 and 24) and 2^21 elements of x (more of them through 64-token tiles cost what the cast saved:
+// 65536 tokens x 128 x 128 17.0 against 13.3, 4096 x 512 x 512 11.5 against 12.5).
+bool small_f32(const Tensor& x, const Tensor& w) {
+    if (!x.is_cuda() || x.device() != w.device() || x.scalar_type() != at::kBFloat16 || w.scalar_type() != at::kFloat ||
+        w.dim() != 2 || x.dim() < 1 || x.size(-1) != w.size(1) || x.layout() != at::kStrided || w.layout() != at::kStrided)
+        return false;
+    const int64_t O = w.size(0), I = w.size(1);
+    if (x.numel() == 0 || O == 0 || O % 4 || I % 8 || I > 2048) return false;
+    return x.numel() <= (1 << 21) && x.numel() <= (int64_t(1) << 30) / O && plain({&x, &w});
+}
+
 struct Linear : torch::autograd::Function<Linear> {
-    static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w) {
+    static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& w, bool small, bool grad) {
+        if (small) {
+            const Tensor xd = dense(x), wd = dense(w);
+            std::vector<int64_t> size(x.sizes().begin(), x.sizes().end());
+            size.back() = w.size(0);
+            const Tensor y = empty(size, at::kBFloat16, x), wc = grad ? empty(w.sizes(), at::kBFloat16, x) : Tensor();
+            check(rwkv6_linear_f32(ptr(xd), fptr(wd), ptr(y), ptr(wc), xd.numel() / w.size(1), w.size(0), w.size(1),
+                                   stream_of(x)),
+                  "rwkv6_linear_f32");
+            if (grad) {
+                ctx->save_for_backward({x, wc});
+                put(ctx, {code(w)});
+            }
+            return y;
+        }
         const Tensor wc = cast(w, x.scalar_type());
         ctx->save_for_backward({x, wc});
         put(ctx, {code(w)});
@@ -541,12 +569,12 @@ struct Linear : torch::autograd::Function<Linear> {
         if (ctx->needs_input_grad(0)) dx = at::mm(dy, wc).view(x.sizes());
         if (ctx->needs_input_grad(1))
             dw = splitk_wgrad(dy, x.reshape({-1, x.size(-1)}).contiguous(), type(meta(ctx)[0]));
-        return {dx, dw};
+        return {dx, dw, Tensor(), Tensor()};
     }
 };
 Tensor linear(const Tensor& x, const Tensor& w) {
     no_transforms();
-    return Linear::apply(x, w);
+    return Linear::apply(x, w, small_f32(x, w), recorded({&x, &w}, OptTensor()));
 }
 
 }  // namespace

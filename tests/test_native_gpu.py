@@ -101,3 +101,30 @@ def test_transforms_are_refused(pkg, name):
     import torch.autograd.forward_ad as fwd
     with fwd.dual_level(), pytest.raises((RuntimeError, NotImplementedError)):
         _outs(fn(fwd.make_dual(leaves[0].clone().requires_grad_(True), torch.ones_like(leaves[0])), *leaves[1:]))
+
+
+# Token tiles of 32 (eight waves: few workgroups; four) and 64, their remainders, a tail of the 64 or 128
+# inputs of a step, outputs that do not fill a tile.  Both operands are exact in bf16, so the result differs
+# from float64's by its own rounding, 2^-9, and the fp32 sums' 2^-23 I sum |x w|; the bf16 weight that the
+# backward multiplies with gives the library path's dx bit for bit.
+@pytest.mark.parametrize("N,O,I", [(1, 4, 8), (31, 64, 64), (32, 68, 72), (33, 200, 712), (65, 60, 2048),
+                                   (1030, 512, 136), (2050, 512, 64), (2112, 516, 200)])
+def test_linear_of_an_fp32_weight(pkg, N, O, I):
+    g = torch.Generator().manual_seed(N + O)
+    x = torch.randn(N, 1, I, generator=g).to(torch.bfloat16).to(DEV).requires_grad_(True)
+    w = (torch.randn(O, I, generator=g) * I ** -0.5).to(DEV).requires_grad_(True)
+    dy = torch.randn(N, 1, O, generator=g).to(torch.bfloat16).to(DEV)
+    linear = pkg._lib.native().linear
+    y = linear(x, w)
+    wb = w.detach().to(torch.bfloat16).requires_grad_(True)
+    ref = x.detach().double() @ wb.detach().double().t()
+    mag = x.detach().double().abs() @ wb.detach().double().abs().t()
+    assert y.shape == (N, 1, O) and y.dtype == torch.bfloat16
+    assert bool(((y.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 2.0 ** -23 * I * mag).all())
+    dx, dw = torch.autograd.grad(y, (x, w), dy)
+    dxb, _ = torch.autograd.grad(linear(x, wb), (x, wb), dy)
+    assert torch.equal(dx, dxb) and dw.dtype == torch.float32 and dw.shape == w.shape
+    with torch.no_grad():
+        assert torch.equal(linear(x, w), y) and torch.equal(linear(x[:1, 0], w), linear(x[:1], w)[0])
+    strided = x.detach().transpose(0, 2).contiguous().transpose(0, 2)
+    assert torch.equal(linear(strided, w), y)
