@@ -202,6 +202,46 @@ def test_group_norm_gate(pkg, head_first, pdt, T, B, H):
     _check("dbeta", _n(leaves[3].grad), dbet)
 
 
+@pytest.mark.parametrize("head_first,gate", [(True, True), (False, True), (False, False)])
+@pytest.mark.parametrize("T,B,H", [(2047, 1, 64), (4097, 2, 32), (4033, 3, 12)])
+def test_group_norm_four_heads(pkg, head_first, gate, T, B, H):
+    """Sizes around the one from which a block takes four heads (512 blocks of 64 tokens in the
+    backward, 1024 in the forward), last tiles of 1 and 63 tokens, head counts that are a multiple of
+    four only; against fp64 on the same inputs.  Outputs: the bf16 rounding (2^-9) and the fp32
+    arithmetic before it; the parameters' sums run over N = T B bf16-exact products in fp32."""
+    if not gate:                                  # the plain GroupNorm reads [N, C]
+        T, B = T * B, 1
+    C = H * 64
+    g = torch.Generator(device=DEV).manual_seed(T + H)
+    rn = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    o = _bf(rn(B, H, T, 64) * 2 + 0.5)
+    if not head_first:
+        o = o.permute(2, 0, 1, 3).reshape(T, B, C).contiguous()
+    leaves = [o, _bf(rn(T, B, C)), 1 + 0.3 * rn(C), 0.2 * rn(C)]
+    dy = _bf(rn(T, B, C))
+    leaves = [t.requires_grad_(True) for t in leaves]
+    wrt = leaves if gate else leaves[:1] + leaves[2:]
+    if gate:
+        y = pkg.timemix.group_norm_gate(*leaves, 1e-5, head_first=head_first)
+    else:
+        y = pkg.timemix.group_norm(leaves[0].view(T, C), H, leaves[2], leaves[3], 1e-5).view(T, B, C)
+    got = [y] + list(torch.autograd.grad(y, wrt, dy))
+    ref = [t.detach().double().requires_grad_(True) for t in leaves]
+    x = ref[0].permute(2, 0, 1, 3).reshape(T, B, C) if head_first else ref[0]
+    x = x.view(T, B, H, 64)
+    x = x - x.mean(-1, keepdim=True)
+    x = x * torch.rsqrt((x * x).mean(-1, keepdim=True) + 1e-5)
+    yr = x.reshape(T, B, C) * ref[2] + ref[3]
+    if gate:
+        yr = yr * torch.nn.functional.silu(ref[1])
+    want = [yr] + list(torch.autograd.grad(yr, ref if gate else ref[:1] + ref[2:], dy.double()))
+    for a, b in zip(got, want):
+        assert a.shape == b.shape
+        assert ((a.double() - b).norm() / b.norm()).item() < 2.0 ** -8
+        # elementwise: half a bf16 unit of the value, and fp32 rounding of terms of the size of the rms
+        assert ((a.double() - b).abs() <= 2.0 ** -8 * b.abs() + 1e-4 * b.square().mean().sqrt()).all()
+
+
 def test_mix_and_gn_deterministic(pkg):
     T, B, C, H = 200, 3, 256, 4
     g = torch.Generator().manual_seed(1)
