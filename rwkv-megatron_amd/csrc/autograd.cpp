@@ -353,7 +353,8 @@ struct LayerNorm : torch::autograd::Function<LayerNorm> {
                                    fptr(copy), N, C, stream_of(x)),
               "rwkv6_layer_norm_fwd");
         if (grad) {
-            ctx->save_for_backward({x, copy.defined() ? copy : gamma, mean, rstd});
+            // the input itself: a dense copy made here has no history for a second derivative
+            ctx->save_for_backward({xi, copy.defined() ? copy : gamma, mean, rstd});
             if (copy.defined()) ctx->saved_data["gamma"] = gamma;
             ctx->saved_data["beta"] = beta;
         }
@@ -361,7 +362,7 @@ struct LayerNorm : torch::autograd::Function<LayerNorm> {
     }
     static variable_list backward(AutogradContext* ctx, variable_list gr) {
         const auto s = ctx->get_saved_variables();
-        const Tensor &x = s[0], &mean = s[2], &rstd = s[3];
+        const Tensor x = dense(s[0]), &mean = s[2], &rstd = s[3];
         const bool own = ctx->saved_data.count("gamma") == 0;       // gamma is the saved tensor itself
         const Tensor gamma = own ? s[1] : ctx->saved_data["gamma"].toTensor(), beta = ctx->saved_data["beta"].toTensor();
         const bool ng = ctx->needs_input_grad(1), nb = ctx->needs_input_grad(2);

@@ -109,3 +109,24 @@ def test_layer_norm_second_derivative_and_updates(modules):
     with torch.no_grad():
         ln.weight.mul_(2)
     assert torch.equal(torch.autograd.grad(y, x, dy)[0], want)
+
+
+# The same chain, so the same bound, for an input that the kernels read through a dense copy: strided, or
+# off the 16-byte grid.  x enters the loss a second time, so that a lost d(dx)/dx would not be an error.
+@pytest.mark.parametrize("form", ["transposed", "shifted"])
+@pytest.mark.parametrize("wdt", [F32, BF])
+def test_layer_norm_second_derivative_of_a_copied_input(modules, form, wdt):
+    ln = _norm(modules, 64, wdt, wdt)
+    x, dy = _case((6, 5), 64)
+    x = x.transpose(0, 1) if form == "transposed" else torch.cat([x.reshape(-1)[:1], x.reshape(-1)])[1:].view(x.shape)
+    dy = dy.transpose(0, 1) if form == "transposed" else dy
+    x = x.detach().requires_grad_(True)
+    assert not x.is_contiguous() or x.data_ptr() % 16
+
+    def second(f):
+        gx, gw = torch.autograd.grad(f(x), (x, ln.weight), dy, create_graph=True)
+        return torch.autograd.grad(gx.float().square().sum() + gw.float().square().sum() + x.float().sum(), (x, ln.weight))
+
+    a, b = second(ln), second(lambda t: F.layer_norm(t, (64,), ln.weight.to(BF), ln.bias.to(BF), ln.eps))
+    for p, q in zip(a, b):
+        assert float((p.float() - q.float()).abs().max()) <= 2.0 ** -5 * float(q.float().abs().max())
