@@ -574,10 +574,12 @@ inline bool al16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) 
 inline size_t lf_round(size_t n) { return (n + 255) & ~(size_t)255; }
 inline bool dt_ok(int d) { return d == RWKV6_F32 || d == RWKV6_BF16; }
 inline int launch_status() { return hipGetLastError() == hipSuccess ? RWKV6_OK : RWKV6_ERR_LAUNCH; }
-// The kernels' bottlenecks; 64 token rows of a batch column within 32-bit byte offsets.
-inline bool lf_supported(int64_t B, int64_t C, int64_t E, int64_t R, bool lerp) {
-    return (lerp ? E == LF_E_MIX && R == LF_R_MIX : E == 1 && R == LF_R_DECAY) && C <= (1 << 23) &&
-           B <= (1 << 23) / C;
+// What the kernels take, the same for the forward, the backward and its workspace: their bottlenecks;
+// 64 token rows of a batch column within 32-bit byte offsets; a grid of 32-token workgroups of 256
+// threads below the launch's 2^32 threads.
+inline bool lf_supported(int64_t T, int64_t B, int64_t C, int64_t E, int64_t R, bool lerp) {
+    return (lerp ? E == LF_E_MIX && R == LF_R_MIX : E == 1 && R == LF_R_DECAY) && C % 64 == 0 && C <= (1 << 23) &&
+           B <= (1 << 23) / C && T <= ((int64_t)1 << 28) / B;
 }
 // Token rows of a workgroup of the down and d_pre kernels.  Each workgroup reads the whole weight,
 // so the mixes' 64 rows halve that traffic once 64 rows a workgroup still give half the CUs one
@@ -614,12 +616,11 @@ int rwkv6_lora_down_fwd(const void* x, const void* maa, int maa_dtype, const voi
     if (T < 0 || B < 1 || C < 1 || E < 1 || R < 1) return RWKV6_ERR_INVALID_ARG;
     if (!dt_ok(w_dtype) || (maa && !dt_ok(maa_dtype))) return RWKV6_ERR_INVALID_ARG;
     const bool lerp = maa != nullptr, f32 = w_dtype == RWKV6_F32;
-    if (C % 64 || !lf_supported(B, C, E, R, lerp)) return RWKV6_ERR_UNSUPPORTED;
+    if (!lf_supported(T, B, C, E, R, lerp)) return RWKV6_ERR_UNSUPPORTED;
     if (T == 0) return RWKV6_OK;
     if (!x || !w_down || !neck) return RWKV6_ERR_INVALID_ARG;
     if (!al16(x) || !al16(maa) || !al16(w_down) || !al16(neck)) return RWKV6_ERR_ALIGNMENT;
     const int64_t N = T * B;
-    if (N > ((int64_t)1 << 36)) return RWKV6_ERR_UNSUPPORTED;          // the grid's range
     if (any_alias({{neck, (size_t)(N * E * R) * 2}},
                   {{x, (size_t)(N * C) * 2}, {maa, (size_t)C * param_bytes(maa_dtype)},
                    {w_down, (size_t)(C * E * R) * param_bytes(w_dtype)}}))
@@ -636,7 +637,7 @@ int rwkv6_lora_down_fwd(const void* x, const void* maa, int maa_dtype, const voi
 }
 
 size_t rwkv6_lora_bwd_workspace_bytes(int64_t T, int64_t B, int64_t C, int64_t E, int64_t R) {
-    if (T < 0 || B < 1 || C < 64 || C % 64 || (E != 1 && E != LF_E_MIX) || !lf_supported(B, C, E, R, E != 1)) return 0;
+    if (T < 0 || B < 1 || C < 1 || !lf_supported(T, B, C, E, R, E != 1)) return 0;
     const LfPlan p = lf_plan(T, B, C, E != 1);
     return lf_round((size_t)(T * B * E * R) * 2) + (size_t)(std::max(p.np, 1) * lf_cols(E, R, C, E != 1)) * 4;
 }
@@ -702,8 +703,7 @@ int rwkv6_lora_bwd(const void* x, const void* maa, int maa_dtype, const void* co
         (maa && !dt_ok(maa_dtype)))
         return RWKV6_ERR_INVALID_ARG;
     const bool lerp = maa != nullptr, f32 = w_dtype == RWKV6_F32;
-    if (C % 64 || B > 65535 || !lf_supported(B, C, E, R, lerp)) return RWKV6_ERR_UNSUPPORTED;
-    if (T > ((int64_t)1 << 30) || T * B > ((int64_t)1 << 36)) return RWKV6_ERR_UNSUPPORTED;
+    if (!lf_supported(T, B, C, E, R, lerp)) return RWKV6_ERR_UNSUPPORTED;
     if (!w_down || !w_up || !bias || !d_w_down || !d_w_up || !d_bias || !workspace || (!d_maa != !maa) ||
         (T > 0 && (!x || !neck || !dx || !d_out)))
         return RWKV6_ERR_INVALID_ARG;

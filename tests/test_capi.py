@@ -117,6 +117,27 @@ def test_overlapping_outputs_are_rejected(pkg):
                                None) == E.RWKV6_ERR_INVALID_ARG
 
 
+@pytest.mark.parametrize("E,R", [(5, 32), (1, 64), (5, 64), (1, 32), (2, 32)])
+def test_bottleneck_calls_agree_on_what_they_take(pkg, E, R):
+    """The backward's workspace query, by which a caller chooses these kernels, is nonzero exactly for
+    the shapes that the forward and the backward take (null tensors: a shape they take is refused for
+    those, after the shape)."""
+    L, e = pkg._lib.load(), pkg._lib
+    maa = _fake(0x100000) if E > 1 else None
+    seen = set()
+    for T in (0, 1, 63, 4096, (1 << 28) - 1, 1 << 28, (1 << 28) + 1, (1 << 30) + 1):
+        for B in (1, 2, 4, 4097, 65535, 65536, 70000, 131072, 131073):
+            for C in (8, 64, 96, 128, 2048, 1 << 23, (1 << 23) + 64):
+                took = L.rwkv6_lora_bwd_workspace_bytes(T, B, C, E, R) != 0
+                want = e.RWKV6_ERR_INVALID_ARG if took else e.RWKV6_ERR_UNSUPPORTED
+                assert L.rwkv6_lora_bwd(None, maa, 0, None, None, None, None, 0, None, 0, None, None, None, 0, None, 0,
+                                        None, None, T, B, C, E, R, None) == want, (T, B, C)
+                if T:
+                    assert L.rwkv6_lora_down_fwd(None, maa, 0, None, 0, None, T, B, C, E, R, None) == want, (T, B, C)
+                seen.add(took)
+    assert seen == ({True, False} if (E, R) in ((5, 32), (1, 64)) else {False})
+
+
 def test_python_checker_maps_codes(pkg):
     with pytest.raises(NotImplementedError):
         pkg._lib.check(2, "x")

@@ -430,3 +430,12 @@ def test_bottleneck_kernels_match_the_general_path(pkg, form, T, B, C, wdt, udt,
         if a.numel():
             err = float((a.double() - c.double()).norm() / c.double().norm().clamp_min(1e-20))
             assert err <= 1.6e-2 or float(c.double().abs().max()) == 0.0 == float(a.double().abs().max()), (i, err)
+
+
+# More batch columns than a grid's second dimension holds; bars as above.
+def test_decay_bottleneck_of_many_batch_columns(pkg):
+    leaves, dy = _bottleneck_case("decay", 1, 70000, 64, torch.bfloat16, torch.bfloat16, torch.bfloat16)
+    got = _bottleneck_run(pkg, "decay", leaves, dy)
+    ref = _bottleneck_run(pkg, "decay", leaves, dy, general=True)
+    for i, (a, c) in enumerate(zip(got, ref)):
+        assert float((a.double() - c.double()).norm()) <= 1.6e-2 * float(c.double().norm()), i
