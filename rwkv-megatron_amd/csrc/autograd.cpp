@@ -523,6 +523,13 @@ Tensor splitk_wgrad(const Tensor& dy, const Tensor& x, at::ScalarType dt) {
     if (s == 1 && (!dy.is_cuda() || dt == dy.scalar_type() || dy.scalar_type() != at::kBFloat16 || N == 0))
         return cast(at::mm(dy.t(), x), dt);
     TORCH_CHECK_TYPE(dy.is_cuda(), "split weight gradients run on the GPU");
+    // A backward that is differentiated itself: bmm with an output type and the summing kernel have no
+    // derivative.  One product in fp32 for a parameter wider than bf16 (exact products, as the batched
+    // one's), else in the operands' type.
+    if (at::GradMode::is_enabled()) {
+        const bool wide = dt != dy.scalar_type() && dy.scalar_type() == at::kBFloat16;
+        return cast(wide ? at::mm(dy.t().to(at::kFloat), x.to(at::kFloat)) : at::mm(dy.t(), x), dt);
+    }
     const Tensor part = at::bmm(dy.view({s, N / s, O}).transpose(1, 2), x.view({s, N / s, I}), at::kFloat);
     return s == 1 ? cast(part.view({O, I}), dt) : sum_partials(part, dt);
 }

@@ -128,3 +128,26 @@ def test_linear_of_an_fp32_weight(pkg, N, O, I):
         assert torch.equal(linear(x, w), y) and torch.equal(linear(x[:1, 0], w), linear(x[:1], w)[0])
     strided = x.detach().transpose(0, 2).contiguous().transpose(0, 2)
     assert torch.equal(linear(strided, w), y)
+
+
+# dx = dy W and dW = dy^T x are linear, so d(sum dW * m)/dx = dy m and so on: exact in bf16 operands up to
+# one rounding, 2^-9, of each bf16 result and the fp32 sums.  One chunk of tokens, odd (N = 33), and a
+# count that the plain backward splits (10240).
+@pytest.mark.parametrize("N", [33, 10240])
+@pytest.mark.parametrize("wdt", [torch.float32, torch.bfloat16])
+def test_linear_second_derivative(pkg, N, wdt):
+    g = torch.Generator().manual_seed(N)
+    bf = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16).to(DEV)
+    x, dy, m = bf(N, 64).requires_grad_(True), bf(N, 32).requires_grad_(True), bf(32, 64)
+    w = (bf(32, 64).float() * 0.125).to(wdt).requires_grad_(True)
+    y = pkg._lib.native().linear(x, w)
+    plain = torch.autograd.grad(y, w, dy.detach(), retain_graph=True)[0]
+    dw = torch.autograd.grad(y, w, dy, create_graph=True)[0]
+    ref = dy.detach().double().t() @ x.detach().double()
+    for t in (plain, dw):
+        assert t.dtype == wdt
+        half = 2.0 ** -8 if wdt == torch.bfloat16 else 0.0
+        assert bool(((t.double() - ref).abs() <= half * ref.abs() + 2.0 ** -23 * N * 16).all())
+    gx, gdy = torch.autograd.grad((dw * m).sum(), (x, dy))
+    for got, want in ((gx, dy.detach().double() @ m.double()), (gdy, x.detach().double() @ m.double().t())):
+        assert bool(((got.double() - want).abs() <= 2.0 ** -7 * want.abs() + 2.0 ** -23 * 64 * 16).all())
