@@ -40,11 +40,14 @@ void check(int status, const char* what) {
     if (status == RWKV6_ERR_UNSUPPORTED) C10_THROW_ERROR(NotImplementedError, msg);
     if (status == RWKV6_ERR_INVALID_ARG || status == RWKV6_ERR_ALIGNMENT) C10_THROW_ERROR(ValueError, msg);
     const std::string full = msg + " (status " + std::to_string(status) + ")";
-    if (g_error && PyGILState_Check()) {
-        PyErr_SetString(g_error, full.c_str());
-        throw py::error_already_set();
-    }
-    throw std::runtime_error(full);
+    if (!g_error) throw std::runtime_error(full);
+    // a backward node runs without the interpreter lock; the exception keeps its Python type on the way
+    // through the autograd engine's threads
+    py::gil_scoped_acquire gil;
+    PyErr_SetString(g_error, full.c_str());
+    python_error e;
+    e.persist();
+    throw e;
 }
 
 void* stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
@@ -589,6 +592,11 @@ Tensor linear(const Tensor& x, const Tensor& w) {
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.attr("ABI_VERSION") = RWKV6_ABI_VERSION;
+    // a status as the functions here raise it, from a thread that does not hold the interpreter lock
+    m.def("check", [](int status, const std::string& what) {
+        py::gil_scoped_release nogil;
+        check(status, what.c_str());
+    });
     m.def("set_error", [](py::object cls) { g_error = cls.release().ptr(); });
     m.def("wkv6", torch::wrap_pybind_function(wkv6));
     m.def("wkv6_seqfirst", torch::wrap_pybind_function(wkv6_seqfirst));

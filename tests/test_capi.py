@@ -148,6 +148,18 @@ def test_python_checker_maps_codes(pkg):
     pkg._lib.check(0, "x")
 
 
+def test_native_checker_maps_codes(pkg):
+    """The C++ functions raise the same types, from a thread without the interpreter lock too (as a
+    backward runs them)."""
+    check, E = pkg._lib.native().check, pkg._lib
+    check(E.RWKV6_OK, "x")
+    for status, kind in ((E.RWKV6_ERR_UNSUPPORTED, NotImplementedError), (E.RWKV6_ERR_INVALID_ARG, ValueError),
+                         (E.RWKV6_ERR_ALIGNMENT, ValueError), (E.RWKV6_ERR_LAUNCH, E.Rwkv6Error)):
+        with pytest.raises(kind, match="^x: ") as e:
+            check(status, "x")
+        assert type(e.value) is kind
+
+
 def test_wrapper_rejects_cpu_tensors(pkg):
     import torch
     x = torch.zeros(1, 1, 4, 64, dtype=torch.bfloat16)
