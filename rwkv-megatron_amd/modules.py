@@ -88,9 +88,15 @@ def _ramp(C, layer_id, n_layers, device):
     return 1.0 - torch.pow(ddd, ratio)
 
 
+def _linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """y = x W^T in x's dtype: on the GPU csrc/autograd.cpp's function, elsewhere plain torch, which
+    needs neither shared library."""
+    return _lib.native().linear(x, w) if x.is_cuda else F.linear(x, w.to(x.dtype))
+
+
 class _Linear(nn.Module):
     """Column/RowParallelLinear at TP=1: weight [out, in], y = x @ W^T, optional bias; the weight
-    gradient split over the tokens (csrc/autograd.cpp).
+    gradient on the GPU split over the tokens (csrc/autograd.cpp).
 
     The weight is initialised by the config's Megatron init callable (``init_attr``:
     ``init_method`` or ``output_layer_init_method``) when it has one, else normal(0, std);
@@ -113,7 +119,7 @@ class _Linear(nn.Module):
                     nn.init.normal_(self.weight, 0.0, std)
 
     def forward(self, x):
-        y = _lib.native().linear(x, self.weight)
+        y = _linear(x, self.weight)
         if self.bias is None:
             return y, None
         b = self.bias.to(y.dtype)
@@ -138,11 +144,11 @@ class LayerNorm(nn.LayerNorm):
 
 class OutputLayer(nn.Linear):
     """The untied output head (rwkv6_model.py, output_layer) as y = x W^T with the parameter cast
-    to the activations' dtype; the weight gradient by the split-token GEMM
-    of csrc/autograd.cpp."""
+    to the activations' dtype; the weight gradient on the GPU by the split-token GEMM of
+    csrc/autograd.cpp."""
 
     def forward(self, x):
-        return _lib.native().linear(x, self.weight)
+        return _linear(x, self.weight)
 
 
 class GroupNorm(nn.Module):

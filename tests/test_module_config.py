@@ -154,3 +154,34 @@ def test_package_config_decay_ramp_still_selectable(pkg):
     tm = M.RWKV6TimeMix(cfg, 1)
     b = tm.bottleneck_decay.bias[0]
     assert abs(b[0].item() + 6.0) < 1e-6 and abs(b[-1].item() + 1.0) < 1e-5
+
+
+@pytest.mark.parametrize("tokens", [5, 8])
+@pytest.mark.parametrize("dtype,wdt", [(torch.float32, torch.float32), (torch.bfloat16, torch.float32)])
+def test_linears_on_the_cpu_need_no_library(pkg, monkeypatch, tokens, dtype, wdt):
+    """The projections and the head of CPU tensors are plain torch: values, both gradients and the
+    weight's dtype, with the shared libraries out of reach.  Operands that are exact in bf16: a result
+    is off by its own rounding, 2^-9, an fp32 one by its sums."""
+    M = pkg.modules
+
+    def missing(*_):
+        raise RuntimeError("not built")
+
+    monkeypatch.setattr(pkg._lib, "native", missing)
+    monkeypatch.setattr(pkg._lib, "load", missing)
+    cfg = megatron_config(params_dtype=wdt)
+    g = torch.Generator().manual_seed(tokens)
+    bf = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16)
+    for m in (M._Linear(cfg, 64, 48, 0.02, "cpu"), M.OutputLayer(64, 48, bias=False, dtype=wdt)):
+        w, x, dy = bf(48, 64), bf(tokens, 1, 64), bf(tokens, 1, 48)
+        with torch.no_grad():
+            m.weight.copy_(w)
+        xi = x.to(dtype).requires_grad_(True)
+        y = m(xi)
+        y = y[0] if isinstance(y, tuple) else y
+        dx, dw = torch.autograd.grad(y, (xi, m.weight), dy.to(dtype))
+        x2, dy2, wd = x.double().view(-1, 64), dy.double().view(-1, 48), w.double()
+        assert y.dtype == dx.dtype == dtype and dw.dtype == wdt
+        for got, want in ((y, x2 @ wd.t()), (dx, dy2 @ wd), (dw, dy2.t() @ x2)):
+            bound = (2.0 ** -8 if dtype == torch.bfloat16 else 0.0) * want.abs() + 2.0 ** -23 * 64 * 16
+            assert bool(((got.double().view(want.shape) - want).abs() <= bound).all())
