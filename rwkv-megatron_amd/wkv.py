@@ -66,10 +66,12 @@ def chunk_rwkv6(r, k, v, g, u, scale=None, initial_state=None, output_final_stat
         raise NotImplementedError("only the head-first [B,H,T,K] layout is supported")
     if scale is None or scale == -1:
         scale = _HEAD ** -0.5
+    scale = float(scale)
     try:
-        out = _lib.native().wkv6(r, k, v, g, u, initial_state, float(scale), bool(output_final_state))
-    except TypeError:
-        out = None
+        out = _lib.native().wkv6(r, k, v, g, u, initial_state, scale, bool(output_final_state))
+    except TypeError:                       # not a tensor: say which; or raised on the way (a hook)
+        _validate(r, k, v, g, u, initial_state)
+        raise
     if out is None:                         # an argument does not fit: say which
         _validate(r, k, v, g, u, initial_state)
         raise ValueError("WKV6 arguments do not fit together")

@@ -56,6 +56,18 @@ def test_saved_tensor_hooks_and_versions(pkg, name):
         torch.autograd.grad(sum(t.float().square().sum() for t in out), leaves)
 
 
+@pytest.mark.parametrize("name", NAMES)
+@pytest.mark.parametrize("kind", [TypeError, ValueError])
+def test_an_error_of_a_saved_tensor_hook_is_raised_itself(pkg, name, kind):
+    fn, leaves = _ops(pkg)[name]
+
+    def pack(t):
+        raise kind("from the hook")
+
+    with torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t), pytest.raises(kind, match="from the hook"):
+        fn(*[t.requires_grad_(True) for t in leaves])
+
+
 @pytest.mark.parametrize("name", ["wkv", "seqfirst", "mix", "lerp"])
 def test_unused_outputs_have_zero_gradients(pkg, name):
     """A loss on one output alone: the same gradients as with zero gradients for the others."""
