@@ -161,6 +161,14 @@ void no_transforms() {
                 "the RWKV-6 kernels' autograd functions do not support torch.func transforms");
 }
 
+// A forward without the interpreter lock, as torch's own operators run: a launch that waits for room
+// in the queue, or an allocation that synchronises, does not stop the program's other threads.
+template <class F>
+auto unlocked(F&& f) {
+    py::gil_scoped_release nogil;
+    return f();
+}
+
 // whether a backward can follow (the condition under which torch records the function)
 bool recorded(std::initializer_list<const Tensor*> ts, const OptTensor& h0) {
     if (!at::GradMode::is_enabled()) return false;
@@ -180,8 +188,9 @@ py::object wkv6(const Tensor& r, const Tensor& k, const Tensor& v, const Tensor&
     if (h0 && (h0->device() != r.device() || h0->sizes() != at::IntArrayRef({r.size(0), r.size(1), 64, 64})))
         return py::none();
     no_transforms();
-    const variable_list out = Wkv6::apply(r, k, v, w, u, h0, scale, (int64_t)0, final_state,
-                                            recorded({&r, &k, &v, &w, &u}, h0));
+    const variable_list out = unlocked([&] {
+        return Wkv6::apply(r, k, v, w, u, h0, scale, (int64_t)0, final_state, recorded({&r, &k, &v, &w, &u}, h0));
+    });
     if (final_state) return py::make_tuple(out[0], out[1]);
     return py::make_tuple(out[0], py::none());
 }
@@ -189,8 +198,9 @@ py::object wkv6(const Tensor& r, const Tensor& k, const Tensor& v, const Tensor&
 py::tuple wkv6_seqfirst(const Tensor& r, const Tensor& k, const Tensor& v, const Tensor& decay, const Tensor& u,
                         const OptTensor& h0, double scale, int64_t heads, bool final_state) {
     no_transforms();
-    const variable_list out = Wkv6::apply(r, k, v, decay, u, h0, scale, heads, final_state,
-                                            recorded({&r, &k, &v, &decay, &u}, h0));
+    const variable_list out = unlocked([&] {
+        return Wkv6::apply(r, k, v, decay, u, h0, scale, heads, final_state, recorded({&r, &k, &v, &decay, &u}, h0));
+    });
     if (final_state) return py::make_tuple(out[0], out[1]);
     return py::make_tuple(out[0], py::none());
 }
@@ -279,13 +289,13 @@ py::object token_shift_mix(const Tensor& x, const Tensor& maa, const Tensor& w_d
                            const Tensor& bias) {
     if (!fits(x, &maa, w_down, w_up, bias)) return py::none();
     no_transforms();
-    const variable_list o = Bottleneck::apply(x, OptTensor(maa), w_down, w_up, bias);
+    const variable_list o = unlocked([&] { return Bottleneck::apply(x, OptTensor(maa), w_down, w_up, bias); });
     return py::make_tuple(o[0], o[1], o[2], o[3], o[4]);
 }
 py::object decay_lora(const Tensor& x, const Tensor& w_down, const Tensor& w_up, const Tensor& bias) {
     if (!fits(x, nullptr, w_down, w_up, bias)) return py::none();
     no_transforms();
-    return py::cast(Bottleneck::apply(x, OptTensor(), w_down, w_up, bias)[0]);
+    return py::cast(unlocked([&] { return Bottleneck::apply(x, OptTensor(), w_down, w_up, bias)[0]; }));
 }
 
 // ---------------------------------------------------------------------------------------
@@ -335,7 +345,7 @@ struct GroupNormGate : torch::autograd::Function<GroupNormGate> {
 Tensor group_norm_gate(const Tensor& o, const OptTensor& g, const Tensor& gamma, const Tensor& beta, double eps,
                        bool head_first) {
     no_transforms();
-    return GroupNormGate::apply(o, g, gamma, beta, eps, head_first);
+    return unlocked([&] { return GroupNormGate::apply(o, g, gamma, beta, eps, head_first); });
 }
 
 // ---------------------------------------------------------------------------------------
@@ -413,7 +423,7 @@ py::object layer_norm(const Tensor& x, const OptTensor& gamma, const OptTensor& 
             (t->scalar_type() != at::kBFloat16 && t->scalar_type() != at::kFloat && t->scalar_type() != at::kHalf))
             return py::none();
     if (!plain({&x, &*gamma, &*beta})) return py::none();
-    return py::cast(LayerNorm::apply(x, *gamma, *beta, eps, recorded({&x, &*gamma}, beta)));
+    return py::cast(unlocked([&] { return LayerNorm::apply(x, *gamma, *beta, eps, recorded({&x, &*gamma}, beta)); }));
 }
 
 // ---------------------------------------------------------------------------------------
@@ -452,7 +462,7 @@ struct CmixLerp : torch::autograd::Function<CmixLerp> {
 };
 py::tuple cmix_lerp(const Tensor& x, const Tensor& mix) {
     no_transforms();
-    const variable_list o = CmixLerp::apply(x, mix);
+    const variable_list o = unlocked([&] { return CmixLerp::apply(x, mix); });
     return py::make_tuple(o[0], o[1]);
 }
 
@@ -471,7 +481,7 @@ struct ReluSq : torch::autograd::Function<ReluSq> {
 };
 Tensor relu_sq(const Tensor& up) {
     no_transforms();
-    return ReluSq::apply(up);
+    return unlocked([&] { return ReluSq::apply(up); });
 }
 
 struct SigmoidGate : torch::autograd::Function<SigmoidGate> {
@@ -492,7 +502,7 @@ struct SigmoidGate : torch::autograd::Function<SigmoidGate> {
 };
 Tensor sigmoid_gate(const Tensor& out, const Tensor& gate_pre) {
     no_transforms();
-    return SigmoidGate::apply(out, gate_pre);
+    return unlocked([&] { return SigmoidGate::apply(out, gate_pre); });
 }
 
 // ---------------------------------------------------------------------------------------
@@ -585,7 +595,7 @@ struct Linear : torch::autograd::Function<Linear> {
 };
 Tensor linear(const Tensor& x, const Tensor& w) {
     no_transforms();
-    return Linear::apply(x, w, small_f32(x, w), recorded({&x, &w}, OptTensor()));
+    return unlocked([&] { return Linear::apply(x, w, small_f32(x, w), recorded({&x, &w}, OptTensor())); });
 }
 
 }  // namespace

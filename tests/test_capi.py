@@ -160,6 +160,34 @@ def test_native_checker_maps_codes(pkg):
         assert type(e.value) is kind
 
 
+def test_a_forward_leaves_the_interpreter_to_other_threads(pkg):
+    """While a function of the extension runs (here one product on the CPU, a hundred milliseconds),
+    another thread goes on: with the lock held it could run once before and once after the call."""
+    import threading
+    import time
+
+    import torch
+
+    x = torch.randn(3000, 3000)
+    count, stop = [0], threading.Event()
+
+    def work():
+        while not stop.is_set():
+            time.sleep(0.001)
+            count[0] += 1
+
+    t = threading.Thread(target=work)
+    t.start()
+    try:
+        before = count[0]
+        pkg._lib.native().linear(x, x)
+        inside = count[0] - before
+    finally:
+        stop.set()
+        t.join()
+    assert inside > 3, inside
+
+
 def test_wrapper_rejects_cpu_tensors(pkg):
     import torch
     x = torch.zeros(1, 1, 4, 64, dtype=torch.bfloat16)
