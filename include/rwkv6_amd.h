@@ -266,7 +266,7 @@ int rwkv6_linear_f32(const void* x, const float* w, void* y, void* w_bf16, int64
 
 /* ------------------------------------------------------------------------
  * LayerNorm over the C channels of N bf16 rows (rwkv6_layer_specs.py:543-547), C a multiple of 8
- * up to 4096 (else RWKV6_ERR_UNSUPPORTED).  gamma, beta: [C] in param_dtype; y: [N,C] bf16;
+ * up to 4096, N at most 2^26 - 4 (else RWKV6_ERR_UNSUPPORTED).  gamma, beta: [C] in param_dtype; y: [N,C] bf16;
  * mean, rstd: [N] f32 for the backward; gamma_copy: [C] f32, nullable: gamma as it was used.
  * ---------------------------------------------------------------------- */
 int rwkv6_layer_norm_fwd(const void* x, const void* gamma, const void* beta, int param_dtype,

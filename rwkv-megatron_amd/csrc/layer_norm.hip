@@ -202,7 +202,8 @@ inline bool al16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) 
 inline int ln_check(int64_t N, int64_t C, int pdt) {
     if (N < 0 || C < 1) return RWKV6_ERR_INVALID_ARG;
     if (pdt != RWKV6_F32 && pdt != RWKV6_BF16) return RWKV6_ERR_INVALID_ARG;
-    if (C % 8 || C > LN_MAX_C || N > (int64_t)1 << 32) return RWKV6_ERR_UNSUPPORTED;
+    // rows: a grid of 256 threads for four of them stays below the launch's 2^32 threads
+    if (C % 8 || C > LN_MAX_C || N > ((int64_t)1 << 26) - 4) return RWKV6_ERR_UNSUPPORTED;
     return RWKV6_OK;
 }
 // Row ranges of the backward: 8 rows (two a wave) at least, so that few rows still spread over the

@@ -138,6 +138,19 @@ def test_bottleneck_calls_agree_on_what_they_take(pkg, E, R):
     assert seen == ({True, False} if (E, R) in ((5, 32), (1, 64)) else {False})
 
 
+def test_layer_norm_takes_the_rows_that_a_launch_covers(pkg):
+    """256 threads for four rows, below 2^32 threads: more rows are refused by the workspace query (by
+    which a module falls back to torch) and by both entries (null tensors are refused after the shape)."""
+    L, e = pkg._lib.load(), pkg._lib
+    for N in (0, 1, (1 << 26) - 4, (1 << 26) - 3, 1 << 26, 1 << 32):
+        took = -(-N // 4) * 256 < 1 << 32
+        assert (L.rwkv6_layer_norm_bwd_workspace_bytes(N, 8) != 0) == took
+        want = e.RWKV6_ERR_INVALID_ARG if took else e.RWKV6_ERR_UNSUPPORTED
+        assert L.rwkv6_layer_norm_bwd(None, None, 0, None, None, None, None, None, None, 0, None, N, 8, None) == want
+        if N:
+            assert L.rwkv6_layer_norm_fwd(None, None, None, 0, 1e-5, None, None, None, None, N, 8, None) == want
+
+
 def test_python_checker_maps_codes(pkg):
     with pytest.raises(NotImplementedError):
         pkg._lib.check(2, "x")
