@@ -386,3 +386,17 @@ def test_wkv_without_gradients(pkg, shape, state):
         o, hT = pkg.wkv6_seqfirst(tb(r), tb(k), tb(v), tb(decay.to(dev)), u, H, scale=scale,
                                   initial_state=h0 if state else None, output_final_state=True)
     _compare(dict(o=_n(o), hT=_n(hT)), ref, ["o", "hT"])
+
+
+# dh0 is an fp32 sum over the tokens of products with one bf16 rounding (r e^G): an error of 2^-8 / sqrt(3)
+# times the mantissa's share, 0.74 for a uniform logarithm, so 1.66e-3 in relative L2, in every form of the
+# backward: one walk, segments that form their own starts, pieces and folds, chunk-parallel.  A second
+# rounding on the way, of the chunks' contributions say, makes it 2.3e-3.
+@pytest.mark.parametrize("shape,plan", [((1, 8, 777), 0), ((1, 1, 512), 0), ((2, 8, 512), -8), ((1, 32, 2048), 8),
+                                        ((5, 33, 300), 1)])
+def test_wkv_state_gradient_is_carried_in_fp32(pkg, shape, plan):
+    B, H, T = shape
+    assert pkg._lib.load().rwkv6_wkv_plan(B, H, T, 1) == plan
+    x = _inputs(B, H, T, seed=T)
+    got, ref = run_gpu(pkg, x, 1.0, True, False)["dh0"], run_oracle(x, 1.0, True, False)["dh0"]
+    assert parity.metrics(got, ref)["l2_rel"] <= 1.8e-3
