@@ -1258,7 +1258,7 @@ wkv6_bwd_fold(const float* __restrict__ dSp, const float* __restrict__ Ap,
 // reverse walk per sequence to fill the device)
 // ---------------------------------------------------------------------------
 // Per (b,h, chunk): dS_loc = s sum_t (r_t e^{G_{t-1}}) dO_t^T [MFMA] and dec = e^{G_63}; then
-// one scan thread per pair of state elements: dS_out(c-1) = dec(c) dS_out(c) + dS_loc(c).  dS_loc is
+// one scan thread per state element: dS_out(c-1) = dec(c) dS_out(c) + dS_loc(c).  dS_loc is
 // handed over in fp32, as the walk carries it: a plan changes the time, not the precision (in bf16 the
 // error of dh0 was 2.25e-3 against the walk's 1.52e-3, of dv 3.35e-3 against 3.24e-3).
 // SEQ: r and w (as pre-activation decay) are sequence-first; dO is head-first.
@@ -1338,48 +1338,43 @@ wkv6_bwd_chunk_dstate(const uint16_t* __restrict__ r, const uint16_t* __restrict
     for (int tj = 0; tj < 4; ++tj) *reinterpret_cast<f32x4*>(out + 16 * tj) = scale * acc[tj];
 }
 
-// A thread carries two adjacent elements of one state row and issues
-// the loads of SCAN_U chunks before it walks them (they do not depend on the carry).
+// dHs[c] = bf16(dS_out(c)) (gradient w.r.t. the state after chunk c); dh0 = dS_out(-1).  One wave per
+// (b,h, state row): the row's decay is uniform, and a single sequence's states spread over 64 CUs (bound
+// by what a CU loads: with blocks of eight rows the scan of one sequence of 512 chunks took 10 us more).
+// The loads of SCAN_U chunks are issued before the wave walks them (they do not depend on the carry).
 #define SCAN_U 32
-#define SCAN_BLK 8                         // blocks per (b,h): 8 x 256 threads x 2 elements
-
-// dHs[c] = bf16(dS_out(c)) (gradient w.r.t. the state after chunk c); dh0 = dS_out(-1).
-__global__ void __launch_bounds__(NTHR)
+__global__ void __launch_bounds__(KD)
 wkv6_state_scan_bwd(const float* __restrict__ dSloc, const float* __restrict__ decay,
                     const float* __restrict__ dhT, uint16_t* __restrict__ dHs,
                     float* __restrict__ dh0, int NT) {
-    const int bh = blockIdx.x / SCAN_BLK;
-    const int e = ((blockIdx.x % SCAN_BLK) * NTHR + threadIdx.x) * 2;
-    const int i = e >> 6;
-    float2 dS = dhT ? *reinterpret_cast<const float2*>(dhT + (size_t)bh * KD * KD + e) : make_float2(0.f, 0.f);
-    const float2* sl = reinterpret_cast<const float2*>(dSloc + (size_t)bh * NT * KD * KD + e);
+    const int bh = blockIdx.x / KD, i = blockIdx.x % KD;
+    const size_t e = (size_t)bh * KD * KD + i * KD + threadIdx.x;
+    float dS = dhT ? dhT[e] : 0.f;
+    constexpr int ST = KD * KD;
+    const size_t end = (size_t)bh * NT * ST + i * KD + threadIdx.x;
     const float* dc = decay + (size_t)bh * NT * KD + i;
-    uint32_t* hs = reinterpret_cast<uint32_t*>(dHs + (size_t)bh * NT * KD * KD + e);
-    constexpr size_t ST = KD * KD / 2;
     int c = NT - 1;
     for (; c - (SCAN_U - 1) >= 0; c -= SCAN_U) {
-        float2 l[SCAN_U];
-        float d[SCAN_U];
+        const float* sl = dSloc + end + (size_t)(c - (SCAN_U - 1)) * ST;
+        uint16_t* hs = dHs + end + (size_t)(c - (SCAN_U - 1)) * ST;
+        const float* d = dc + (size_t)(c - (SCAN_U - 1)) * KD;
+        float l[SCAN_U], f[SCAN_U];
 #pragma unroll
-        for (int q = 0; q < SCAN_U; ++q) {
-            l[q] = sl[(c - q) * ST];
-            d[q] = dc[(c - q) * KD];
+        for (int q = SCAN_U - 1; q >= 0; --q) {
+            l[q] = sl[q * ST];
+            f[q] = d[q * KD];
         }
 #pragma unroll
-        for (int q = 0; q < SCAN_U; ++q) {
-            hs[(c - q) * ST] = pk2(dS.x, dS.y);
-            dS.x = d[q] * dS.x + l[q].x;
-            dS.y = d[q] * dS.y + l[q].y;
+        for (int q = SCAN_U - 1; q >= 0; --q) {
+            hs[q * ST] = f2bf(dS);
+            dS = f[q] * dS + l[q];
         }
     }
     for (; c >= 0; --c) {
-        hs[c * ST] = pk2(dS.x, dS.y);
-        const float2 l = sl[c * ST];
-        const float d = dc[c * KD];
-        dS.x = d * dS.x + l.x;
-        dS.y = d * dS.y + l.y;
+        dHs[end + (size_t)c * ST] = f2bf(dS);
+        dS = dc[(size_t)c * KD] * dS + dSloc[end + (size_t)c * ST];
     }
-    if (dh0) *reinterpret_cast<float2*>(dh0 + (size_t)bh * KD * KD + e) = dS;
+    if (dh0) dh0[e] = dS;
 }
 
 
@@ -3044,8 +3039,8 @@ int wkv_bwd_impl(const void* r, const void* k, const void* v, const void* w, con
                        scale, (int)B, (int)H, (int)T, (int)NT);
     mark(phase_events, 1, s);
     mark(phase_events, 2, s);
-    hipLaunchKernelGGL(wkv6_state_scan_bwd, dim3((unsigned)BH * SCAN_BLK), dim3(NTHR), 0, s, dSloc,
-                       dec, dhT, dHs, dh0, (int)NT);
+    hipLaunchKernelGGL(wkv6_state_scan_bwd, dim3((unsigned)BH * KD), dim3(KD), 0, s, dSloc, dec, dhT, dHs,
+                       dh0, (int)NT);
     mark(phase_events, 3, s);
     mark(phase_events, 4, s);
     hipLaunchKernelGGL(wkv6_bwd_chunk_grads<SEQ>, dim3((unsigned)NT, (unsigned)BH), dim3(NTHR_G),
