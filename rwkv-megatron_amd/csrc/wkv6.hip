@@ -372,17 +372,24 @@ inline Pieces prepass_pieces(int64_t BH, int64_t NT, int P, int64_t max_pieces) 
 // T = 4096), and where segments start from: `pre`: each forms its start state itself from the
 // chunks before it (backward: after it), else (P > 1) a pre-pass of pieces and a fold do.  P = 0
 // (backward only): the chunk-parallel form.
-// The plan is the fastest by a model in microseconds, fitted to kernels timed on MI355X over
-// B*H = 8..128 and 2..128 chunks (back to back, without launch gaps):
+// The plan is the fastest by a model in microseconds, fitted to kernels timed on MI355X: the walks over
+// B*H = 8..128 and 2..128 chunks, chunk-parallel over B*H = 1..24 and 8..768 chunks (back to back, without
+// launch gaps):
 //   a walk                    chunk us for each chunk of the longest segment
 //   pre                       head + step us for each 128 tokens of the longest prefix
 //   pre-pass (two launches)   9.5 + 0.4 a piece of the sequence + 1.6 for each 128 tokens of a piece
-//   chunk-parallel (four)     12.8 + 0.029 a (b,h, chunk), over what a walk needs besides its chunks
-// (a launch beyond the walk's own is counted as 2 us).  E.g., one segment -> plan: forward of 16
-// sequences of 8 chunks 22.5 -> 15.0 us (pre, 8 segments), of 32 sequences of 32 chunks 34.8 ->
-// 28.3 (pre-pass, 8 segments of 4 chunks instead of 4 of 8); backward of the same 43.9 -> 20.4
-// (pre; chunk-parallel 18.9 with two launches more) and 57.2 -> 42.1, of 8 sequences of 13 chunks
-// 66.5 -> 19.9 (chunk-parallel).
+//   chunk-parallel (four)     11 + 0.03 a (b,h, chunk) + 0.065 a chunk (the scan takes a sequence's one
+//                             after the other), over what a walk needs besides its chunks
+// (a launch beyond the walk's own is counted as 2 us).  Chunk-parallel against the walk, us: 1 sequence
+// of 128 chunks 25 and 40, of 768 79 and 82; 2 of 256 42 and 54, of 512 70 and 72; 4 of 128 35 and 44, of
+// 256 58 and 58; 8 of 13 21.0 and 22.5, of 64 31 and 37, of 128 51 and 49; 16 of 16 24 and 28, of 64 47 and
+// 45; 20 of 20 32 and 30.  Up to eight chunks the two are level (8 sequences of 8: 18.7 and 18.5) and the
+// walk needs two launches fewer.  From 129 sequences on the walk is one segment: chunk-parallel was 286
+// against 309 us at 129 sequences of 64 chunks and level at 144, for 24 KB of workspace a (b,h, chunk),
+// 1.8 GB at 144 sequences of 512 chunks, where the walk takes 256 bytes a sequence.
+// One segment -> plan: forward of 16 sequences of 8 chunks 22.5 -> 15.0 us (pre, 8 segments), of 32
+// sequences of 32 chunks 34.8 -> 28.3 (pre-pass, 8 segments of 4 chunks instead of 4 of 8); backward of
+// the same 43.9 -> 20.4 (pre) and 57.2 -> 42.1, of 8 sequences of 13 chunks 66.5 -> 21.1 (chunk-parallel).
 struct WalkPlan {
     int P;
     bool pre;
@@ -417,7 +424,8 @@ inline WalkPlan fwd_walk_plan(int64_t BH, int64_t NT) {
 inline WalkPlan bwd_walk_plan(int64_t BH, int64_t NT) {
     double cost;
     const WalkPlan p = walk_plan(BH, NT, BWD_MODEL, &cost);
-    return NT < 2 || cost <= 12.8 + 0.029 * (double)(BH * NT) ? p : WalkPlan{0, false};
+    if (BH > WALK_TARGET_ITEMS / 2 || NT <= 8) return p;
+    return cost <= 11 + 0.03 * (double)(BH * NT) + 0.065 * (double)NT ? p : WalkPlan{0, false};
 }
 
 struct WalkPrefetch {

@@ -60,6 +60,23 @@ def test_workspace_sizes(pkg):
     assert L.rwkv6_wkv_saved_bytes(B, H, T, 32, 64) == 0          # unsupported head size
 
 
+def test_backward_plans_of_long_and_many_sequences(pkg):
+    """The chunk-parallel backward serves few sequences of a bounded number of chunks: with more
+    sequences than half the CUs each is one walk whatever its length, whose workspace holds the du
+    partials alone, and one or a few very long sequences are walked in segments (the scan over the
+    chunks is serial).  Both keep the workspace far below a state a chunk."""
+    L = pkg._lib.load()
+    for BH in (129, 132, 144, 150, 158, 200, 256, 1000):
+        for NT in (1, 15, 29, 64, 512, 4096):
+            assert L.rwkv6_wkv_plan(1, BH, 64 * NT, 1) == 1
+            assert L.rwkv6_wkv_workspace_bytes(1, BH, 64 * NT, 64, 64, 1) <= 256 * BH + 256
+    for BH in (1, 2, 4, 7, 8, 64, 128):
+        for NT in (1024, 2048, 4096):
+            assert L.rwkv6_wkv_plan(1, BH, 64 * NT, 1) > 1
+            assert L.rwkv6_wkv_workspace_bytes(1, BH, 64 * NT, 64, 64, 1) < 24 << 20
+    assert L.rwkv6_wkv_plan(1, 8, 64 * 32, 1) == 0 == L.rwkv6_wkv_plan(1, 1, 64 * 512, 1)
+
+
 def _fake(addr):
     return ctypes.c_void_p(addr)
 

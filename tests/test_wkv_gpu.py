@@ -392,7 +392,7 @@ def test_wkv_without_gradients(pkg, shape, state):
 # times the mantissa's share, 0.74 for a uniform logarithm, so 1.66e-3 in relative L2, in every form of the
 # backward: one walk, segments that form their own starts, pieces and folds, chunk-parallel.  A second
 # rounding on the way, of the chunks' contributions say, makes it 2.3e-3.
-@pytest.mark.parametrize("shape,plan", [((1, 8, 777), 0), ((1, 1, 512), 0), ((2, 8, 512), -8), ((1, 32, 2048), 8),
+@pytest.mark.parametrize("shape,plan", [((1, 8, 777), 0), ((1, 1, 640), 0), ((2, 8, 512), -8), ((1, 32, 2048), 8),
                                         ((5, 33, 300), 1)])
 def test_wkv_state_gradient_is_carried_in_fp32(pkg, shape, plan):
     B, H, T = shape
@@ -417,3 +417,16 @@ def test_wkv_error_does_not_depend_on_the_plan(pkg, shape, plan):
     for k in ("dr", "dk", "dv", "dw", "dh0"):
         a, b = (parity.metrics(t, ref[k])["l2_rel"] for t in (got[k], walk[k][:, :H]))
         assert a <= 1.01 * b, (k, a, b)
+
+
+# Both sides of the backward's line between the walk and the chunk-parallel form: up to eight chunks, the
+# length from which few sequences are walked in segments, one walk each from 129 sequences on.
+@pytest.mark.parametrize("shape,plan", [((1, 4, 512), -8), ((1, 4, 577), 0), ((2, 2, 64 * 170 - 5), 0),
+                                        ((2, 2, 64 * 250 - 5), 63), ((1, 128, 1000), -2), ((3, 43, 1000), 1),
+                                        ((1, 1, 64 * 800 + 1), 0), ((1, 1, 64 * 1024 + 1), 147)])
+def test_wkv_backward_forms(pkg, shape, plan):
+    B, H, T = shape
+    assert pkg._lib.load().rwkv6_wkv_plan(B, H, T, 1) == plan
+    x = _inputs(B, H, T, seed=T)
+    got, ref = run_gpu(pkg, x, 0.5, True, True), run_oracle(x, 0.5, True, True)
+    _compare(got, ref, ["o", "hT", "dr", "dk", "dv", "dw", "du", "dh0"])
