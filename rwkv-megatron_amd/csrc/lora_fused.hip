@@ -272,9 +272,13 @@ rwkv6_lora_dpre_kernel(const uint16_t* __restrict__ x, InPtrs<E> dout,
     }
 }
 
-// The rest of the backward.  Workgroup (pidx, cb): the 64 channels c0 = 64 cb of the token tiles
-// of one range (and, LERP, one batch column: a tile is 64 consecutive tokens t of batch b, so
-// the shift is one row).  Per tile
+// The rest of the backward.  Workgroup (pidx, cb): the 64 channels c0 = 64 cb of one range of the token
+// tiles.  A tile is 64 rows of all tokens; LERP, 64 consecutive tokens t of one batch column b, so that
+// the shift is one row, or (T <= 32) `cpt` whole columns of T rows each, row r being token t = r mod T of
+// column r / T.  A range walks its tiles across the columns' ends, so that the number of ranges, each of
+// which writes a full set of partial gradients, follows the device and not the batch (a range per column
+// wrote 684 MB at [64, 256, 2048] and took 833 us forward and backward; now 21 MB and 398 us; [1, 4096,
+// 2048] 7157 -> 139 us).  Per tile
 //   m_e = neck_e W_up_e (LERP), d_xxx = d_pre W_down^T                     [MFMA, to fp32 tiles]
 //   dm_e = d_out_e (shift(x) - x),  d_delta = sum_e d_out_e (m_e + bias_e) + d_xxx maa
 //   dx[t] = sum_e d_out_e + d_xxx - d_delta[t] + d_delta[t+1]   (E = 1: dx = d_xxx)
@@ -310,7 +314,7 @@ rwkv6_lora_grads_kernel(const uint16_t* __restrict__ x, const void* __restrict__
                         const uint16_t* __restrict__ dpre, const void* __restrict__ wup,
                         const void* __restrict__ wd, const void* __restrict__ bias, int bdt,
                         uint16_t* __restrict__ dxo, float* __restrict__ part, int64_t T, int64_t B,
-                        int64_t C, int ntiles, int tpr, int nr, int np) {
+                        int64_t C, int ntiles, int cpt, int tiles, int tpr, int np) {
     constexpr int ER = E * R, WS = ER + 8, NA = ER / 32, KS = R / 32;
     constexpr int STEP = LERP ? LF_TT - 1 : LF_TT;
     constexpr int NP = LF_TT * ER / 8, NPT = (NP + LF_THR - 1) / LF_THR;
@@ -320,8 +324,7 @@ rwkv6_lora_grads_kernel(const uint16_t* __restrict__ x, const void* __restrict__
     // their channel blocks, so neck and d_pre of a range are read into one L2
     const int ncb = (int)(C / 64), id = blockIdx.x, pidx = (id >> 3) / ncb * 8 + (id & 7), cb = (id >> 3) % ncb;
     if (pidx >= np) return;
-    const int64_t b = pidx / nr;
-    const int t_lo = (pidx - (int)b * nr) * tpr, t_hi = min(ntiles, t_lo + tpr);
+    const int t_lo = pidx * tpr, t_hi = min(tiles, t_lo + tpr);
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, L = lane & 15, q = lane >> 4;
     const int ct = wv & 3, hh = wv >> 2, cg = tid & 7;
     const int64_t c0 = 64 * (int64_t)cb;
@@ -351,6 +354,17 @@ rwkv6_lora_grads_kernel(const uint16_t* __restrict__ x, const void* __restrict__
     for (int ks = 0; ks < NA; ++ks)
         wda[ks] = __builtin_bit_cast(bf16x8, w_bf16<WF32>(w_load<WF32>(wd, (c0 + 16 * ct + L) * ER + 32 * ks + 8 * q)));
 
+    // Tile g: its first token t0 and column b0, its rows, and whether the sequences end in it.
+    struct Tile { int64_t t0, b0; int rows; bool end; };
+    auto tile = [&](int g) {
+        const int col = LERP ? g / ntiles : 0, ti = g - col * ntiles;
+        const int64_t t0 = (int64_t)ti * STEP, b0 = (int64_t)col * cpt;
+        const int rows = LERP && cpt > 1 ? min(cpt, (int)(B - b0)) * (int)T : (int)min<int64_t>(LF_TT, T - t0);
+        return Tile{t0, b0, rows, ti == ntiles - 1};
+    };
+    // (column, token) of a tile's row, after b0 and t0: r / T by a factor rounded up, exact for r < 64
+    const unsigned inv = LERP && cpt > 1 ? (65536u + (unsigned)T - 1) / (unsigned)T : 0u;
+    auto col_of = [&](int r) { return LERP ? (int)((unsigned)r * inv >> 16) : 0; };
     // Addresses: a wave-uniform base per tile plus 32-bit byte offsets of the thread (B*C is
     // bounded by lf_supported, so that 64 token rows fit); rows past the end read the last token.
     uint4 xr, pr, dq[E], nkr[NPT], dpr[NPT];
@@ -358,26 +372,23 @@ rwkv6_lora_grads_kernel(const uint16_t* __restrict__ x, const void* __restrict__
     auto at = [](const uint16_t* p, unsigned bytes) {
         return *reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(p) + bytes);
     };
-    auto load_rows = [&](int ti, int tid) {          // neck, d_pre
-        const int64_t t0 = (int64_t)ti * STEP, base = (t0 * B + b) * ER;
-        const int last = (int)min<int64_t>(LF_TT, T - t0) - 1;
+    auto load_rows = [&](const Tile& tl, int tid) {          // neck, d_pre
+        const int64_t base = (tl.t0 * B + tl.b0) * ER;
 #pragma unroll
         for (int i = 0; i < NPT; ++i) {
-            const int p = min(tid + LF_THR * i, NP - 1), rw = p / (ER / 8);
-            const unsigned o = (unsigned)min(rw, last) * rsn + 16 * (p - rw * (ER / 8));
+            const int p = min(tid + LF_THR * i, NP - 1), rw = p / (ER / 8), r = min(rw, tl.rows - 1), c = col_of(r);
+            const unsigned o = (unsigned)(r - c * (int)T) * rsn + (unsigned)c * (2 * ER) + 16 * (p - rw * (ER / 8));
             nkr[i] = at(neck + base, o);
             dpr[i] = at(dpre + base, o);
         }
     };
-    auto load_acts = [&](int ti, int tid) {
-        const int row = tid >> 3, cg = tid & 7;
-        const int64_t t0 = (int64_t)ti * STEP, base = (t0 * B + b) * C + c0;
-        const int last = (int)min<int64_t>(LF_TT, T - t0) - 1;
-        const int rw = min(row, last);
-        const unsigned o = (unsigned)rw * rs + 16 * cg;
+    auto load_acts = [&](const Tile& tl, int tid) {
+        const int cg = tid & 7, r = min(tid >> 3, tl.rows - 1), c = col_of(r), t = r - c * (int)T;
+        const int64_t base = (tl.t0 * B + tl.b0) * C + c0;
+        const unsigned o = (unsigned)t * rs + (unsigned)c * (2 * (unsigned)C) + 16 * cg;
         xr = at(x + base, o);
         // token t - 1; token 0 reads itself (and its shift is zeroed where it is used)
-        if (LERP) pr = at(x + (t0 > 0 ? base - B * C : base), t0 > 0 || rw == 0 ? o : o - rs);
+        if (LERP) pr = at(x + (tl.t0 > 0 ? base - B * C : base), tl.t0 > 0 || t == 0 ? o : o - rs);
 #pragma unroll
         for (int e = 0; e < E; ++e) dq[e] = at(dout.p[e] + base, o);
     };
@@ -388,8 +399,9 @@ rwkv6_lora_grads_kernel(const uint16_t* __restrict__ x, const void* __restrict__
     for (int e = 0; e < E; ++e) ab[e] = 0.f;
     constexpr int DMR = LERP ? LF_MS * 4 : LF_TS * 2;         // bytes of a dm row
     if (t_lo < t_hi) {
-        load_rows(t_lo, threadIdx.x);
-        load_acts(t_lo, threadIdx.x);
+        const Tile tl = tile(t_lo);
+        load_rows(tl, threadIdx.x);
+        load_acts(tl, threadIdx.x);
     }
     for (int ti = t_lo; ti < t_hi; ++ti) {
         // the lane indices from an opaque copy per tile: hoisted out of the walk, the addresses
@@ -400,9 +412,11 @@ rwkv6_lora_grads_kernel(const uint16_t* __restrict__ x, const void* __restrict__
         const int ct = wv & 3, hh = wv >> 2, row = tid >> 3, cg = tid & 7;
         // byte offset of the 4-channel chunk 4 (L & 3) of channel tile ct in a dm row
         const int dmc = LERP ? (2 * ct + ((L & 3) >> 1)) * 32 + (L & 1) * 8 : (16 * ct + 4 * (L & 3)) * 2;
-        const int64_t tr = (int64_t)ti * STEP + row;
+        const Tile tl = tile(ti);
+        const int col = col_of(row), tw = row - col * (int)T;
+        const int64_t tr = tl.t0 + tw;
         // counted here: the tile's own tokens (all of them in the sequence's last tile)
-        const bool cnt = tr < T && (!LERP || row < STEP || ti == ntiles - 1);
+        const bool cnt = row < tl.rows && (!LERP || row < STEP || tl.end);
         __syncthreads();                             // the previous tile's operands are read
 #pragma unroll
         for (int i = 0; i < NPT; ++i) {
@@ -481,7 +495,7 @@ rwkv6_lora_grads_kernel(const uint16_t* __restrict__ x, const void* __restrict__
         }
         // the next tile's loads (the last tile reloads itself), then this tile's weight-gradient
         // products and dx
-        const int tn = min(ti + 1, t_hi - 1);
+        const Tile tn = tile(min(ti + 1, t_hi - 1));
         load_rows(tn, tid);
         load_acts(tn, tid);
         if (LERP) {
@@ -508,7 +522,9 @@ rwkv6_lora_grads_kernel(const uint16_t* __restrict__ x, const void* __restrict__
                 adn[i] = mfma32(xa, lds_tr8(&sm.dp[0][0], WS, 32 * ks, r0, lane), adn[i]);
             }
         }
-        if (cnt) store8(dxo + ((int64_t)ti * STEP * B + b) * C + c0 + (size_t)((unsigned)row * rs / 2 + 8 * cg), dxv);
+        if (cnt)
+            store8(dxo + (tl.t0 * B + tl.b0) * C + c0 + (size_t)((unsigned)tw * (rs / 2) + (unsigned)col * (unsigned)C + 8 * cg),
+                   dxv);
     }
     // ---- partial parameter gradients of the range ----
     float* po = part + (int64_t)pidx * lf_cols(E, R, C, LERP);
@@ -587,23 +603,26 @@ inline bool lf_supported(int64_t T, int64_t B, int64_t C, int64_t E, int64_t R, 
 // decay's smaller weight, 32 rows spread a short walk over twice the CUs (N = 1024, C = 512:
 // mixes 18 -> 12.4 and 13.4 -> 10.9 us, decay 6.9 -> 5.0 and 9.1 -> 5.5).
 inline int lf_tile(int64_t N, bool lerp) { return lerp && N > 8192 ? 64 : 32; }
-// Tiles, tiles a range and ranges of the gradient kernel.  The time is the rounds of
-// workgroups over the device times the tiles of a range; fewer ranges (less partial traffic)
-// win ties.  `slots`: workgroups the device holds at once (LDS: one LERP workgroup of 157 KB a
-// CU, two of the decay's).
-struct LfPlan { int ntiles, tpr, nr, np; };
+// Tiles of the gradient kernel: `ntiles` a batch column (or a group of `cpt` columns of at most 32 tokens,
+// which fill a tile together), `tiles` in all, `np` ranges of `tpr`.  The time is the rounds of workgroups
+// over the device times the tiles of a range; the fewest rounds (and so the least partial traffic) win
+// ties.  `slots`: workgroups the device holds at once (LDS: one LERP workgroup of 157 KB a CU, two of the
+// decay's).  At most 64 ranges for each of up to four columns: more are not measured.
+struct LfPlan { int ntiles, cpt, tiles, tpr, np; };
 inline LfPlan lf_plan(int64_t T, int64_t B, int64_t C, bool lerp) {
-    const int64_t rows = lerp ? T : T * B, nb = lerp ? B : 1, ncb = C / 64, slots = lerp ? 256 : 512;
-    const int64_t nt = rows <= 0 ? 0 : lerp ? (rows > 1 ? (rows - 1 + LF_TT - 2) / (LF_TT - 1) : 1)
-                                            : (rows + LF_TT - 1) / LF_TT;
-    if (nt == 0) return {0, 1, 1, 0};
+    if (T * B == 0) return {0, 1, 0, 1, 0};
+    const int64_t ncb = C / 64, slots = lerp ? 256 : 512;
+    const int64_t cpt = lerp && T <= LF_TT / 2 ? std::min(B, LF_TT / T) : 1, groups = lerp ? (B + cpt - 1) / cpt : 1;
+    const int64_t nt = lerp ? (T > 1 ? (T - 1 + LF_TT - 2) / (LF_TT - 1) : 1) : (T * B + LF_TT - 1) / LF_TT;
+    const int64_t tiles = groups * nt, most = std::min(tiles, 64 * (lerp ? std::min<int64_t>(B, 4) : 1));
     int64_t best = 1, cost = INT64_MAX;
-    for (int64_t nr = 1; nr <= nt && nr <= 64; ++nr) {
-        const int64_t tpr = (nt + nr - 1) / nr, c = ((ncb * nb * nr + slots - 1) / slots) * (tpr + 1);
-        if (c < cost) { cost = c; best = nr; }
+    for (int64_t k = 1; k <= 4; ++k) {
+        const int64_t np = std::max<int64_t>(1, std::min(most, k * slots / ncb));
+        const int64_t c = ((ncb * np + slots - 1) / slots) * ((tiles + np - 1) / np + 1);
+        if (c < cost) { cost = c; best = np; }
     }
-    const int64_t tpr = (nt + best - 1) / best, nr = (nt + tpr - 1) / tpr;
-    return {(int)nt, (int)tpr, (int)nr, (int)(nb * nr)};
+    const int64_t tpr = (tiles + best - 1) / best;
+    return {(int)nt, (int)cpt, (int)tiles, (int)tpr, (int)((tiles + tpr - 1) / tpr)};
 }
 
 }  // namespace
@@ -681,7 +700,7 @@ int lora_bwd_launch(const uint16_t* x, const void* maa, int mdt, const InPtrs<E>
                            dpre, N, B, C);
         hipLaunchKernelGGL(kg, dim3((unsigned)(8 * ((p.np + 7) / 8) * (C / 64))), dim3(LF_THR),
                            sizeof(GradsSmem<E, R, LERP>), s, x, maa, mdt, dout, neck, (const uint16_t*)dpre, wup, wd,
-                           bias, bdt, dx, part, LERP ? T : N, LERP ? B : (int64_t)1, C, p.ntiles, p.tpr, p.nr, p.np);
+                           bias, bdt, dx, part, LERP ? T : N, LERP ? B : (int64_t)1, C, p.ntiles, p.cpt, p.tiles, p.tpr, p.np);
     }
     hipLaunchKernelGGL(rwkv6_lora_reduce_kernel, dim3((unsigned)((n / 4 + 255) / 256)), dim3(256), 0, s,
                        (const float*)part, p.np, n, outs);

@@ -155,6 +155,21 @@ def test_bottleneck_calls_agree_on_what_they_take(pkg, E, R):
     assert seen == ({True, False} if (E, R) in ((5, 32), (1, 64)) else {False})
 
 
+def test_bottleneck_workspace_follows_the_device(pkg):
+    """The token shift's backward keeps a full set of fp32 partial parameter gradients for each of a
+    number of ranges that fills the device, (2 160 + 6) C floats each, whatever the batch: eight at C =
+    2048, and d_pre of the tokens."""
+    L = pkg._lib.load()
+    part = 326 * 2048 * 4
+    for N, shapes in ((16384, [(4096, 4), (256, 64), (64, 256), (32, 512), (16, 1024), (4, 4096)]),
+                      (4096, [(1, 4096), (2, 2048), (33, 124), (4096, 1)])):
+        for T, B in shapes:
+            n = L.rwkv6_lora_bwd_workspace_bytes(T, B, 2048, 5, 32)
+            assert part <= n - T * B * 160 * 2 <= 8 * part + 256, (T, B, n)
+    # narrow layers: at most 256 ranges
+    assert L.rwkv6_lora_bwd_workspace_bytes(1, 131072, 64, 5, 32) <= 131072 * 320 + 256 * 326 * 64 * 4 + 256
+
+
 def test_layer_norm_takes_the_rows_that_a_launch_covers(pkg):
     """256 threads for four rows, below 2^32 threads: more rows are refused by the workspace query (by
     which a module falls back to torch) and by both entries (null tensors are refused after the shape)."""

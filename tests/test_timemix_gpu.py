@@ -439,3 +439,41 @@ def test_decay_bottleneck_of_many_batch_columns(pkg):
     ref = _bottleneck_run(pkg, "decay", leaves, dy, general=True)
     for i, (a, c) in enumerate(zip(got, ref)):
         assert float((a.double() - c.double()).norm()) <= 1.6e-2 * float(c.double().norm()), i
+
+
+def _bottleneck_exact(form, leaves, dy):
+    """The same outputs and gradients in plain torch in 64 bits."""
+    x, maa, wd, wu, bias = (t.detach().double().requires_grad_(True) for t in leaves)
+    T, B, C = x.shape
+    E, R = wd.shape[1:]
+    delta = torch.cat([torch.zeros_like(x[:1]), x[:-1]]) - x
+    xxx = x + delta * maa if form == "mix" else x
+    neck = torch.tanh(xxx @ wd.reshape(C, E * R)).view(T, B, E, R)
+    m = [neck[:, :, e] @ wu[e] + bias[e] for e in range(E)]
+    out = [x + delta * t for t in m] if form == "mix" else m
+    wrt = [x, maa, wd, wu, bias] if form == "mix" else [x, wd, wu, bias]
+    return [t.detach() for t in out] + list(torch.autograd.grad(out, wrt, [t.double() for t in dy]))
+
+
+# Against 64 bits.  A rounding to bf16 is 2^-8 / sqrt(3) of the value times the mantissa's share, 0.74: 1.66e-3
+# in relative L2.  An output has three on its way (xxx, the neck, itself), a gradient five (xxx, the neck, dm,
+# d_pre, itself); the weights are exact in bf16 here.  Batch columns that share a tile (T <= 32: whole and
+# with rows left over, a last tile of fewer columns), that fill half of one, one row more than a tile, ranges
+# that go on from one column to the next, and enough of each that a range holds several tiles.
+@pytest.mark.parametrize("form", ["mix", "decay"])
+@pytest.mark.parametrize("T,B,C,wdt,pdt", [
+    (1, 1, 64, torch.bfloat16, torch.float32), (1, 4096, 128, torch.bfloat16, torch.bfloat16),
+    (2, 33, 64, torch.float32, torch.float32), (3, 1000, 192, torch.bfloat16, torch.bfloat16),
+    (16, 260, 64, torch.bfloat16, torch.bfloat16), (21, 7, 64, torch.float32, torch.bfloat16),
+    (31, 65, 128, torch.bfloat16, torch.bfloat16), (32, 300, 512, torch.bfloat16, torch.bfloat16),
+    (33, 129, 64, torch.bfloat16, torch.float32), (63, 40, 64, torch.bfloat16, torch.bfloat16),
+    (64, 257, 128, torch.float32, torch.bfloat16), (65, 200, 2048, torch.bfloat16, torch.bfloat16),
+    (130, 90, 64, torch.bfloat16, torch.bfloat16), (700, 3, 2048, torch.bfloat16, torch.bfloat16)])
+def test_bottleneck_kernels_match_float64(pkg, form, T, B, C, wdt, pdt):
+    leaves, dy = _bottleneck_case(form, T, B, C, wdt, wdt, pdt)
+    got = _bottleneck_run(pkg, form, leaves, dy)
+    again = _bottleneck_run(pkg, form, leaves, dy)
+    for i, (a, b, c) in enumerate(zip(got, again, _bottleneck_exact(form, leaves, dy))):
+        assert a.shape == c.shape and torch.equal(a, b)
+        err = float((a.double() - c).norm() / c.norm().clamp_min(1e-20))
+        assert err <= (3 if i < len(dy) else 5) * 1.66e-3 or not c.any(), (i, err)
