@@ -867,6 +867,7 @@ __device__ __forceinline__ void piece_steps(PieceSmem& sm, PieceLoads& nx, int n
 // (lq, lr) of wave (W, hh) gets S[16W + lr][32hh + 16tp + 4lq + rr].  All of the walk's 512
 // threads; LDS is free again after it.
 #define PST 68             // row stride (floats) of the fp32 state handed through LDS
+static_assert(KD * PST * sizeof(float) <= sizeof(PieceSmem), "the handed state fits");
 template <bool SEQ>
 __device__ __forceinline__ void fwd_prefix(unsigned char* smem, const uint16_t* __restrict__ k,
                                            const uint16_t* __restrict__ v,
@@ -1954,6 +1955,8 @@ struct LoopSmem {
     tile_t Out[4];                  // dr, dk, dv, dw staged channel-major (token-major for SEQ)
 };
 static_assert(sizeof(LoopSmem) <= 160 * 1024, "one loop workgroup per CU");
+static_assert(sizeof(PieceSmem) <= sizeof(LoopSmem), "bwd_suffix runs the piece steps in the loop's LDS");
+static_assert((KD * PST + KD) * sizeof(float) <= sizeof(LoopSmem), "and hands the state gradient and decay over in it");
 
 // (J, W) of block b in the order b = W(W+1)/2 + J, J <= W (wave-uniform).
 __device__ __forceinline__ void tri_pair(int b, int& hi, int& lo) {

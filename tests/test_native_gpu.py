@@ -163,3 +163,30 @@ def test_linear_second_derivative(pkg, N, wdt):
     gx, gdy = torch.autograd.grad((dw * m).sum(), (x, dy))
     for got, want in ((gx, dy.detach().double() @ m.double()), (gdy, x.detach().double() @ m.double().t())):
         assert bool(((got.double() - want).abs() <= 2.0 ** -7 * want.abs() + 2.0 ** -23 * 64 * 16).all())
+
+
+# The weight gradient's chunks of tokens: one, two and four of them, on both sides of each line (a chunk of
+# 2560 tokens for few output tiles, of 4096 for more than 32; counts that do not divide), for every parameter
+# type.  Exact bf16 operands: off by the result's own rounding and that of the fp32 sums, N additions to sums
+# of up to 4 sqrt(N), 2^-24 each like a random walk: 2^-22 N, and four times that as the bound.
+@pytest.mark.parametrize("N,O,I,chunks", [
+    (5119, 256, 256, 1), (5118, 256, 256, 1), (5120, 256, 256, 2), (5121, 256, 256, 1), (10238, 256, 256, 2),
+    (10240, 256, 256, 4), (10242, 256, 256, 2), (20480, 200, 72, 4), (8190, 2048, 1280, 1),
+    (8192, 2048, 1280, 2), (8193, 2048, 1280, 1), (16384, 1280, 2048, 4)])
+@pytest.mark.parametrize("wdt", [torch.bfloat16, torch.float32, torch.float16])
+def test_linear_weight_gradient(pkg, N, O, I, chunks, wdt):
+    tiles = -(-O // 256) * -(-I // 256)
+    least, s = 4096 if tiles > 32 else 2560, 1
+    while s < 4 and tiles * s < 256 and N % (2 * s) == 0 and N // (2 * s) >= least:
+        s *= 2
+    assert s == chunks                                     # the rule of csrc/autograd.cpp, restated
+    g = torch.Generator(device=DEV).manual_seed(N + O)
+    x = torch.randn(N, I, generator=g, device=DEV).to(torch.bfloat16)
+    dy = torch.randn(N, O, generator=g, device=DEV).to(torch.bfloat16)
+    w = (torch.randn(O, I, generator=g, device=DEV) * I ** -0.5).to(wdt).requires_grad_(True)
+    grads = [torch.autograd.grad(pkg._lib.native().linear(x, w), w, dy)[0] for _ in range(2)]
+    ref = dy.double().t() @ x.double()
+    assert grads[0].dtype == wdt and torch.equal(*grads)
+    half = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -10, torch.float32: 0.0}[wdt]
+    bound = half * ref.abs() + 2.0 ** -20 * N
+    assert bool(((grads[0].double() - ref).abs() <= bound).all())

@@ -120,10 +120,21 @@ def test_wkv_extreme_decay_is_floored(pkg):
     _compare(got, ref, ["o", "hT", "dr", "dk", "dv", "dw", "du", "dh0"])
 
 
-@pytest.mark.parametrize("shape", [(2, 2, 200), (4, 6, 64 * 24 + 3), (2, 64, 64 * 17 + 5)])
-def test_wkv_deterministic(pkg, shape):
-    """Bit-identical reruns: the chunk-parallel backward (B*H = 4 and 24) and, at B*H = 128,
-    the segmented forward and reverse walks (their pieces and folds sum in a fixed order)."""
+def _plans(pkg, shape):
+    """rwkv6_wkv_plan of the forward and the backward: segments a sequence (negative: they form their own
+    start states), 0 the chunk-parallel backward."""
+    L = pkg._lib.load()
+    return L.rwkv6_wkv_plan(*shape, 0), L.rwkv6_wkv_plan(*shape, 1)
+
+
+@pytest.mark.parametrize("shape,plans", [
+    ((2, 2, 200), (-4, -4)), ((4, 6, 64 * 24 + 3), (9, 9)), ((2, 64, 64 * 17 + 5), (-2, -2)),
+    ((2, 2, 64 * 12 + 3), (-13, 0)), ((2, 64, 64 * 64 + 5), (2, 2))])
+def test_wkv_deterministic(pkg, shape, plans):
+    """Bit-identical reruns: segments that form their own start states, segments started by pieces and
+    folds (which sum in a fixed order), the chunk-parallel backward, and pieces and folds of 128
+    sequences in segments of an odd number of chunks (33 and 32)."""
+    assert _plans(pkg, shape) == plans
     x = _inputs(*shape, seed=3)
     a = run_gpu(pkg, x, 1.0, True, True)
     b = run_gpu(pkg, x, 1.0, True, True)
@@ -143,23 +154,21 @@ def test_wkv_empty_sequence(pkg):
     assert torch.equal(hT, h0)
 
 
-@pytest.mark.parametrize("shape", [(1, 2, 1100), (1, 1, 64 * 40 + 17), (2, 24, 64 * 32 + 11),
-                                   (3, 32, 64 * 20), (2, 8, 64 * 64), (1, 32, 64 * 15 + 40),
-                                   (2, 64, 64 * 17 + 5), (1, 128, 64 * 30 + 9),
-                                   (1, 1, 64 * 72 + 10), (1, 1, 64 * 64 + 30)])
-def test_wkv_parity_segmented(pkg, shape):
-    """Few sequences of many chunks: the forward cuts each sequence into segments (pre-pass
-    pieces folded into each segment's start state, then output walks), here 2 segments of 9
-    chunks, 5 of 9 with a ragged last chunk, 4 of 9 (48 sequences), 2 of 10 (96 sequences),
-    8 of 8 (16 sequences) and 2 of 8 with a ragged last chunk (32 sequences).  The backward
-    runs chunk-parallel for those six (the (b,h, segment) walks would fill less than 7/8 of the
-    device: 2, 5, 192, 192, 128 and 64 of 256) and as a segmented reverse walk (backward pieces
-    folded into each segment's starting state gradient) for the 128-sequence shapes: 2
-    segments of 9 chunks, and of 16 + 15 chunks with a ragged last one.  The pieces step two
-    chunks at a time, so segments of an odd chunk count (9, 15) end on a one-chunk step.
-    The last two shapes end the forward on a one-chunk (ragged, 10 tokens) and a two-chunk
-    segment (9 and 8 segments of 9 chunks): the walk's decay scan runs two chunks ahead, so
-    there its look-ahead stays on the segment's last chunk from the start."""
+@pytest.mark.parametrize("shape,plans", [
+    ((1, 2, 1100), (-18, 0)), ((1, 1, 64 * 40 + 17), (21, 0)), ((2, 24, 64 * 32 + 11), (5, 5)),
+    ((3, 32, 64 * 20), (-2, -2)), ((2, 8, 64 * 64), (16, 16)), ((1, 32, 64 * 15 + 40), (-8, 8)),
+    ((2, 64, 64 * 17 + 5), (-2, -2)), ((1, 128, 64 * 30 + 9), (-2, -2)), ((1, 1, 64 * 72 + 10), (19, 0)),
+    ((1, 1, 64 * 64 + 30), (22, 0)), ((1, 64, 64 * 40 + 7), (4, 4)), ((2, 64, 64 * 64 + 5), (2, 2))])
+def test_wkv_parity_segmented(pkg, shape, plans):
+    """Sequences cut into segments, in every form.  Segments that form their own start states: of one
+    chunk (18 a sequence), of two (16 chunks of 32 sequences), of 10 and 9 and an odd count of 16 and 15
+    (128 sequences).  Segments started by the pre-pass, its pieces folded into each segment's start: of 2
+    chunks with a one-chunk ragged last one (41 chunks in 21), of 7 (33 in 5), 4 (16 sequences), 4 and 3,
+    11 (41 in 4, 64 sequences) and 33 and 32 (128 sequences): the pieces step two chunks at a time, so an
+    odd count ends on a one-chunk step, and the walk's decay scan runs two chunks ahead, so a last segment
+    of one or two chunks (73 in 19 of 4, 65 in 22 of 3) stays on its last chunk from the start.  The
+    backward runs chunk-parallel for one and two sequences, as the same forms of the reverse walk else."""
+    assert _plans(pkg, shape) == plans
     B, H, T = shape
     x = _inputs(B, H, T, seed=T)
     got = run_gpu(pkg, x, 0.5, True, True)
@@ -255,14 +264,17 @@ def test_wkv_decay_gradient_through_exp_past_the_floor(pkg):
     _compare(got, ref, ["o", "dr", "dk", "dv", "d_decay", "du"])
 
 
-@pytest.mark.parametrize("shape", [(2, 2, 63), (3, 2, 130), (1, 3, 64), (2, 1, 1300), (2, 24, 2059),
-                                   (2, 64, 1093)])
-def test_wkv_seqfirst_entry(pkg, shape):
+@pytest.mark.parametrize("shape,plans", [
+    ((2, 2, 63), (1, 1)), ((3, 2, 130), (-3, -3)), ((1, 3, 64), (1, 1)), ((2, 1, 1300), (-21, 0)),
+    ((2, 24, 2059), (5, 5)), ((2, 64, 1093), (-2, -2)), ((2, 64, 4101), (2, 2))])
+def test_wkv_seqfirst_entry(pkg, shape, plans):
     """The time-mix module's entry: r, k, v, decay in [T,B,H*64], w = -exp(decay) inside,
     o head-first; d_decay = dw * w.  Checked against the oracle on the rearranged inputs.
-    (2, 24, 2059): B*H = 48, 4 forward segments of 9 chunks and the chunk-parallel backward;
-    (2, 64, 1093): B*H = 128, the segmented walks (2 segments of 9 chunks, ragged end), with
-    scale 0.5 (the other shapes take RWKV-6's unit scale)."""
+    One segment; segments that form their own start states (three of one chunk, 128 sequences in two of
+    9, ragged end); the chunk-parallel backward (two sequences of 21 chunks); pieces and folds (48
+    sequences in 5 segments of 7 chunks, 128 in two of 33 and 32).  128 sequences with scale 0.5 (the
+    other shapes take RWKV-6's unit scale)."""
+    assert _plans(pkg, shape) == plans
     B, H, T = shape
     K = 64
     scale = 0.5 if H == 64 else 1.0

@@ -2,7 +2,7 @@
 rwkv6_wkv_fwd on the same inputs through the C ABI: o, the final state and the saved chunk
 states must be bit-identical (same kernels; only where the pre-pass keeps its segment states
 differs).  Two calls in a row, the second with a smaller input, both on shapes whose forward
-runs the segment pre-pass (B*H < 256), so the library's scratch array carries data; the second
+runs the segment pre-pass, so the library's scratch array carries data; the second
 call finds the first call's contents there.  The outputs are also checked against the CPU
 oracle (max_rel / l2_rel 1e-2)."""
 import ctypes
@@ -16,9 +16,9 @@ from oracle import oracle as orc
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
-# (B, H, T, with h0): 32 chunks in 4 segments x 16 sequences (48 segment states in the
-# scratch array), then 18 chunks in 2 segments x 4 sequences (4 segment states)
-CALLS = [(2, 8, 2000, True), (1, 4, 1100, False)]
+# (B, H, T, with h0): 32 chunks in 16 segments x 16 sequences (240 segment states in the
+# scratch array), then 27 chunks in 14 segments x 4 sequences (52 segment states)
+CALLS = [(2, 8, 2000, True), (1, 4, 1700, False)]
 
 
 def _inputs(B, H, T, seed):
@@ -49,6 +49,10 @@ def _forward(pkg, noalloc, r, k, v, w, u, h0):
     pkg._lib.check(st, "wkv forward")
     torch.cuda.synchronize()
     return o.cpu(), hT.cpu(), saved.cpu()
+
+
+def test_calls_use_the_scratch_array(pkg):
+    assert [pkg._lib.load().rwkv6_wkv_plan(*c[:3], 0) for c in CALLS] == [16, 14]
 
 
 def test_noalloc_forward_matches_workspace_forward(pkg):
