@@ -179,7 +179,8 @@ int rwkv6_shift_lerp_bwd(const void* x, const void* maa, int param_dtype, const 
  *       mixes x + (shift(x) - x) * (neck_e @ w_up[e] + bias[e]) as outputs;
  *   maa (x of the up call) NULL:       E = 1, R = 64, out = neck @ w_up + bias.
  * Other E, R return RWKV6_ERR_UNSUPPORTED (rwkv6_shift_lerp_fwd / rwkv6_ddlerp_lora_* /
- * rwkv6_lora_bias_fwd and GEMMs cover them).  C must be a multiple of 64.
+ * rwkv6_lora_bias_fwd and GEMMs cover them).  C must be a multiple of 64, B*C at most 2^23, T*B at
+ * most 2^28; the workspace query is 0 for what forward and backward refuse.
  *   down: neck [N, E*R] bf16 = tanh(xxx @ w_down)   (or x @ w_down)
  *   up:   out = host array of E device pointers, [T,B,C] bf16 each
  *   bwd:  d_out = host array of E device pointers [T,B,C] bf16; dx [T,B,C] bf16, d_maa [C]

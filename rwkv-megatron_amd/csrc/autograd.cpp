@@ -4,10 +4,11 @@
 // sizes of a small model or a short prompt, and a Python autograd function with its ctypes call
 // cost 40-80 us a direction.
 //
-// Every function keeps no state between calls; tensors it needs again go through
-// save_for_backward (version checks, saved-tensor hooks and checkpointing apply), kernels run on
-// the current stream of the tensors' device, and a backward that reaches a function from
-// forward-mode differentiation or a function transform is refused by torch.
+// Every function keeps no state between calls; tensors whose values it needs again go through
+// save_for_backward (version checks, saved-tensor hooks and checkpointing apply; LayerNorm's
+// backward works on its own copy of a parameter wider than bf16 and keeps the parameters beside it
+// for their types and for a second derivative), kernels run on the current stream of the tensors'
+// device, and a call from forward-mode differentiation or a function transform is refused.
 //
 // Mathematics and reference lines: wkv.py, timemix.py, channelmix.py and modules.py, whose
 // functions check their arguments and call these.

@@ -21,7 +21,7 @@
 // all tokens of a channel.  Reading d_out and x twice (12 x 2C bytes a token) and recomputing
 // m = neck W_up costs less than passing dm ([5,N,C]), the two lerp sums, xxx and d_xxx through
 // HBM between a kernel per step and the library's batched GEMMs of 32 columns.  Measured at N =
-// 16384, C = 2048, forward and backward: the token shift 718 -> 400 us (18 -> 5 launches), the
+// 16384, C = 2048, forward and backward: the token shift 718 -> 390 us (18 -> 5 launches), the
 // decay 391 -> 127 us (16 -> 5); the general path (other ranks) is in timemix.py.
 #include <algorithm>
 #include <utility>
